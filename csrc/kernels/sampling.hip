@@ -4,10 +4,8 @@
 //                              argmax_v (z_v / T + g_v), g_v = -log(-log u_v),
 //                              u_v = hash(seed, step, v)  (counter-based: reproducible per request,
 //                              graph-capturable, no RNG state).  No sort: the top-k and top-p
-//                              thresholds are found by bisection over value with block reductions.
+//                              thresholds come from a histogram of the row (select_threshold).
 // The hash matches mxserve/ops/reference.py::_hash_u32 bit for bit.
-#include <cstdlib>
-
 #include "common.h"
 
 namespace mxs {
@@ -77,210 +75,262 @@ __device__ __forceinline__ float gumbel2(uint32_t key, int v) {
 }
 constexpr float kSLog2e = 1.4426950408889634f;
 
-template <typename T>
-__global__ void __launch_bounds__(1024) sample_kernel(int64_t* __restrict__ out, const T* __restrict__ logits,
-                                                      int V, long row_stride, const float* __restrict__ temperature,
+// ---- a row's logits, wherever they are.  each(f) calls f(logit, index) for every logit this thread owns (slots past the
+// row: -inf with an index >= V).  Register forms: the workgroup loads its row ONCE, 8 neighbouring logits per thread and
+// step of 1024 threads, and every pass runs on registers; rows that do not fit or are not 16-byte aligned are read again
+// by each pass.
+template <int NE>
+struct RegRow16 {  // bf16, packed pairs
+  using T = bf16_t;
+  uint32_t r[NE / 2];
+  __device__ __forceinline__ RegRow16(const bf16_t* z, int V, bool) {
+#pragma unroll
+    for (int q = 0; q < NE / 8; ++q) {
+      const int v0 = 8 * (static_cast<int>(threadIdx.x) + 1024 * q);
+      uint4 w = make_uint4(0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u);  // -inf pairs
+      if (v0 < V) w = *reinterpret_cast<const uint4*>(z + v0);
+      r[4 * q] = w.x;
+      r[4 * q + 1] = w.y;
+      r[4 * q + 2] = w.z;
+      r[4 * q + 3] = w.w;
+    }
+  }
+  template <class F>
+  __device__ __forceinline__ void each(F f) {
+    // an empty asm "modifying" the packed row at the top of each pass: keeps hipcc from carrying all unpacked
+    // floats from one pass to the next, which would spill
+#pragma unroll
+    for (int i = 0; i < NE / 2; ++i) asm volatile("" : "+v"(r[i]));
+    int first = 8 * static_cast<int>(threadIdx.x);
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      if ((e & 7) == 0) asm volatile("" : "+v"(first));  // nor all indices
+      f((e & 1) ? bf2f_hi(r[e >> 1]) : bf2f_lo(r[e >> 1]), first + 8192 * (e >> 3) + (e & 7));
+      if ((e & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // a few independent chains in flight, not the whole row
+    }
+  }
+};
+
+template <int NE>
+struct RegRow32 {
+  using T = float;
+  float r[NE];
+  __device__ __forceinline__ RegRow32(const float* z, int V, bool) {
+#pragma unroll
+    for (int q = 0; q < NE / 8; ++q) {
+      const int v0 = 8 * (static_cast<int>(threadIdx.x) + 1024 * q);
+      float x[8] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY};
+      if (v0 < V) ld8(z, v0, x);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) r[8 * q + i] = x[i];
+    }
+  }
+  template <class F>
+  __device__ __forceinline__ void each(F f) {
+#pragma unroll
+    for (int i = 0; i < NE; ++i) asm volatile("" : "+v"(r[i]));
+    int first = 8 * static_cast<int>(threadIdx.x);
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      if ((e & 7) == 0) asm volatile("" : "+v"(first));
+      f(r[e], first + 8192 * (e >> 3) + (e & 7));
+      if ((e & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+};
+
+template <typename T_>
+struct MemRow {
+  using T = T_;
+  const T* z;
+  int V;
+  bool vec;
+  __device__ __forceinline__ MemRow(const T* z_, int V_, bool vec_) : z(z_), V(V_), vec(vec_) {}
+  template <class F>
+  __device__ __forceinline__ void each(F f) {
+    if (vec) {
+      for (int v = 8 * static_cast<int>(threadIdx.x); v < V; v += 8 * 1024) {
+        float x[8];
+        ld8(z, v, x);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) f(x[u], v + u);
+      }
+    } else {
+      for (int v = threadIdx.x; v < V; v += 1024) f(ld(z, v), v);
+    }
+  }
+};
+
+// Thresholds of the top-k / top-p sets.  "The largest logit x with weight({z >= x}) >= target", weight 1 for top-k and
+// the logit's share of the softmax for top-p, is found from a histogram of weights over kSelBins equal steps of [lo, hi]:
+// the bin in which the sum from the top reaches the target is known after one pass, its logits (some hundred of a
+// 128k row) are collected and ranked against each other; a fuller bin is cut again.  Two passes over the row where a
+// bisection over value took 32, each with an exponential per logit: that was what a row's time went into, and a row is
+// one workgroup, so a step with few sampled rows waits for it (MI355X, 128,256 bf16 logits, 13 rows: 275 us; 32,000
+// fp32 logits, 64 rows: 177 us.  Now 82 us and 27 us).  Weights are 2^-32 fixed point summed in 64-bit integers (shares
+// are at most 1): the sums do not depend on the order of the LDS atomics, so a request's tokens stay reproducible, and
+// they are closer to the exact ones than fp32 sums.
+constexpr int kSelBins = 2048, kSelList = 512;
+struct SelLds {
+  unsigned long long hist[kSelBins];
+  unsigned long long wave[16];
+  unsigned long long above;
+  unsigned long long lw[kSelList];
+  float list[kSelList];
+  int n, bin;
+};
+
+// by_share: weight 2^32 exp2((x - mx) * invt2), target `goal` of the whole; otherwise weight 1, target goal itself.
+// lo <= hi finite; logits outside [lo, hi] have no weight.  -inf when even all of them stay below the target.
+template <class Row>
+__device__ __forceinline__ float select_threshold(Row& R, SelLds& L, float* sv, bool by_share, double goal, float mx,
+                                                  float invt2, float lo, float hi) {
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  auto weight = [&](float x) -> unsigned long long {
+    return by_share ? static_cast<unsigned long long>(static_cast<uint32_t>(
+                          fmaf(__builtin_amdgcn_exp2f((x - mx) * invt2), 4294967040.f, 0.5f)))
+                    : 1ull;
+  };
+  unsigned long long above = 0, target = 0;
+  for (int level = 0; level < 8; ++level) {
+    if (!(hi > lo)) return lo;
+    __syncthreads();  // the level before is done with the bins
+    for (int i = tid; i < kSelBins; i += 1024) L.hist[i] = 0;
+    if (tid == 0) {
+      L.n = 0;
+      L.bin = -1;
+    }
+    __syncthreads();
+    const float scale = fminf(kSelBins / (hi - lo), 3e38f);
+    auto bin_of = [&](float x) -> int {
+      return min(static_cast<int>(fminf((hi - x) * scale, static_cast<float>(kSelBins))), kSelBins - 1);
+    };
+    R.each([&](float x, int) {
+      if (x >= lo && x <= hi) atomicAdd(&L.hist[bin_of(x)], weight(x));
+    });
+    __syncthreads();
+    // the bin that reaches the target: sums from the top, two bins a thread
+    const unsigned long long a = L.hist[2 * tid], b = L.hist[2 * tid + 1];
+    unsigned long long s = a + b;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const unsigned long long t = __shfl_up(s, o, 64);
+      if (lane >= o) s += t;
+    }
+    if (lane == 63) L.wave[wid] = s;
+    __syncthreads();
+    unsigned long long before = above, total = 0;
+#pragma unroll 2
+    for (int w = 0; w < 16; ++w) {
+      if (w < wid) before += L.wave[w];
+      total += L.wave[w];
+    }
+    if (level == 0) {
+      const double t = by_share ? ceil(goal * static_cast<double>(total)) : goal;
+      target = t < 1.0 ? 1ull : static_cast<unsigned long long>(t);
+    }
+    const unsigned long long e0 = before + s - a - b, e1 = e0 + a;
+    if (e0 < target && e1 >= target) {
+      L.bin = 2 * tid;
+      L.above = e0;
+    } else if (e1 < target && e1 + b >= target) {
+      L.bin = 2 * tid + 1;
+      L.above = e1;
+    }
+    __syncthreads();
+    const int bin = L.bin;
+    if (bin < 0) return -INFINITY;
+    above = L.above;
+    // its logits
+    float bmn = INFINITY, bmx = -INFINITY;
+    R.each([&](float x, int) {
+      const bool in = x >= lo && x <= hi && bin_of(x) == bin;
+      const unsigned long long m = __ballot(in);
+      if (m != 0) {
+        const int first = __builtin_ctzll(m);
+        int at = 0;
+        if (lane == first) at = atomicAdd(&L.n, static_cast<int>(__popcll(m)));
+        at = __shfl(at, first, 64) + __popcll(m & ((1ull << lane) - 1));
+        if (in) {
+          bmn = fminf(bmn, x);
+          bmx = fmaxf(bmx, x);
+          if (at < kSelList) L.list[at] = x;
+        }
+      }
+    });
+    __syncthreads();
+    const int n = L.n;
+    if (n <= kSelList) {
+      if (tid < n) L.lw[tid] = weight(L.list[tid]);
+      __syncthreads();
+      float best = -INFINITY;
+      if (tid < n) {
+        const float x = L.list[tid];
+        unsigned long long sum = above;
+#pragma unroll 4
+        for (int j = 0; j < n; ++j) sum += L.list[j] >= x ? L.lw[j] : 0ull;
+        if (sum >= target) best = x;
+      }
+      return block_max(best, sv);
+    }
+    lo = -block_max(-bmn, sv);
+    hi = block_max(bmx, sv);
+  }
+  return lo;
+}
+
+template <class Row>
+__global__ void __launch_bounds__(1024) sample_kernel(int64_t* __restrict__ out,
+                                                      const typename Row::T* __restrict__ logits, int V, long row_stride,
+                                                      bool vec, const float* __restrict__ temperature,
                                                       const float* __restrict__ top_p, const int* __restrict__ top_k,
                                                       const int64_t* __restrict__ seeds,
                                                       const int64_t* __restrict__ steps) {
   __shared__ float sv[16];
   __shared__ int si[16];
+  __shared__ SelLds L;
   const int row = blockIdx.x;
-  const T* z = logits + row * row_stride;
+  Row R(logits + row * row_stride, V, vec);
   const float t = temperature[row];
-  // vectorised single pass when rows are 16-byte aligned (every vocab in the registry)
-  const bool vec = (V % 8 == 0) && (row_stride % 8 == 0) && ((reinterpret_cast<uintptr_t>(logits) & 15) == 0);
   if (!(t > 0.f)) {
     ArgMax a{-INFINITY, 0x7FFFFFFF};
-    if (vec) {
-      for (int v = 8 * threadIdx.x; v < V; v += 8 * blockDim.x) {
-        float x[8];
-        ld8(z, v, x);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) a = better(a, ArgMax{x[u], v + u});
-      }
-    } else {
-      for (int v = threadIdx.x; v < V; v += blockDim.x) a = better(a, ArgMax{ld(z, v), v});
-    }
-    ArgMax r = block_argmax(a, sv, si);
+    R.each([&](float x, int v) {
+      if (v < V) a = better(a, ArgMax{x, v});
+    });
+    const ArgMax r = block_argmax(a, sv, si);
     if (threadIdx.x == 0) out[row] = r.i;
     return;
   }
-  const float invt = 1.f / t;
+  const float invt = 1.f / t, invt2 = invt * kSLog2e;
   const int k = top_k[row];
   const float p = top_p[row];
   float thr = -INFINITY;
   if ((k > 0 && k < V) || p < 1.f) {
     float mx = -INFINITY, mn = INFINITY;
-    for (int v = threadIdx.x; v < V; v += blockDim.x) {
-      mx = fmaxf(mx, ld(z, v));
-      mn = fminf(mn, ld(z, v));
-    }
-    mx = block_max(mx, sv);
-    mn = -block_max(-mn, sv);
-    if (k > 0 && k < V) {  // largest tau with count(z >= tau) >= k
-      float lo = mn, hi = mx;
-      for (int it = 0; it < 32; ++it) {
-        const float mid = 0.5f * (lo + hi);
-        float cnt = 0.f;
-        for (int v = threadIdx.x; v < V; v += blockDim.x) cnt += ld(z, v) >= mid ? 1.f : 0.f;
-        cnt = block_sum(cnt, sv);
-        if (cnt >= static_cast<float>(k)) lo = mid; else hi = mid;
-      }
-      thr = lo;
-    }
-    if (p < 1.f) {  // largest tau with mass(z >= tau) >= p * total, mass in softmax(z / T)
-      float tot = 0.f;
-      for (int v = threadIdx.x; v < V; v += blockDim.x) tot += __expf((ld(z, v) - mx) * invt);
-      tot = block_sum(tot, sv);
-      float lo = fmaxf(mn, mx - 88.f * t), hi = mx;
-      for (int it = 0; it < 32; ++it) {
-        const float mid = 0.5f * (lo + hi);
-        float mass = 0.f;
-        for (int v = threadIdx.x; v < V; v += blockDim.x) {
-          const float zv = ld(z, v);
-          mass += zv >= mid ? __expf((zv - mx) * invt) : 0.f;
-        }
-        mass = block_sum(mass, sv);
-        if (mass >= p * tot) lo = mid; else hi = mid;
-      }
-      thr = fmaxf(thr, lo);
-    }
-  }
-  const uint32_t key = hash_u32(static_cast<uint32_t>(static_cast<uint64_t>(seeds[row]) * 0x9E3779B1ull +
-                                                      static_cast<uint64_t>(steps[row])));
-  const float invt2 = invt * kSLog2e;
-  ArgMax a{-INFINITY, 0x7FFFFFFF};
-  if (vec) {
-    for (int v = 8 * threadIdx.x; v < V; v += 8 * blockDim.x) {
-      float x[8];
-      ld8(z, v, x);
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (x[u] >= thr) a = better(a, ArgMax{x[u] * invt2 + gumbel2(key, v + u), v + u});
-    }
-  } else {
-    for (int v = threadIdx.x; v < V; v += blockDim.x) {
-      const float zv = ld(z, v);
-      if (zv >= thr) a = better(a, ArgMax{zv * invt2 + gumbel2(key, v), v});
-    }
-  }
-  ArgMax r = block_argmax(a, sv, si);
-  if (threadIdx.x == 0) out[row] = r.i;
-}
-
-// Register-resident form (bf16 rows up to 2048 * NV logits, 16-byte aligned): the workgroup loads
-// its row ONCE into registers (NV packed bf16 pairs per thread, 8 consecutive logits per 16-byte
-// load), and every bisection pass of the top-k / top-p thresholds, the max / min and the final
-// Gumbel-max run on those registers.  The memory form above re-reads the row (256 KB at a 128k
-// vocab) for each of up to 64 bisection passes.  Element e of a thread is logit
-// 8 (tid + 1024 (e / 8)) + e % 8; slots past V hold -inf and are skipped.
-template <int NV>
-__global__ void __launch_bounds__(1024) sample_reg_kernel(int64_t* __restrict__ out, const bf16_t* __restrict__ logits,
-                                                          int V, long row_stride, const float* __restrict__ temperature,
-                                                          const float* __restrict__ top_p, const int* __restrict__ top_k,
-                                                          const int64_t* __restrict__ seeds,
-                                                          const int64_t* __restrict__ steps) {
-  constexpr int NQ = NV / 4;  // 16-byte loads per thread
-  constexpr int NE = 2 * NV;  // logits per thread
-  __shared__ float sv[16];
-  __shared__ int si[16];
-  const int row = blockIdx.x, tid = threadIdx.x;
-  const bf16_t* z = logits + row * row_stride;
-  uint32_t r[NV];
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    const int v0 = 8 * (tid + 1024 * q);
-    uint4 w = make_uint4(0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u, 0xFF80FF80u);  // -inf pairs
-    if (v0 < V) w = *reinterpret_cast<const uint4*>(z + v0);
-    r[4 * q] = w.x;
-    r[4 * q + 1] = w.y;
-    r[4 * q + 2] = w.z;
-    r[4 * q + 3] = w.w;
-  }
-  auto val = [&](int e) -> float { return (e & 1) ? bf2f_hi(r[e >> 1]) : bf2f_lo(r[e >> 1]); };
-  // an empty asm "modifying" the packed row at the top of each pass: keeps hipcc from hoisting all
-  // 2 NV unpacked floats out of the bisection loops (loop-invariant), which would spill
-  auto opaque = [&] {
-#pragma unroll
-    for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(r[i]));
-  };
-  auto idx = [&](int e) -> int { return 8 * (tid + 1024 * (e >> 3)) + (e & 7); };
-  const float t = temperature[row];
-  if (!(t > 0.f)) {
-    ArgMax a{-INFINITY, 0x7FFFFFFF};
-#pragma unroll
-    for (int e = 0; e < NE; ++e)
-      if (idx(e) < V) a = better(a, ArgMax{val(e), idx(e)});
-    ArgMax res = block_argmax(a, sv, si);
-    if (tid == 0) out[row] = res.i;
-    return;
-  }
-  const float invt = 1.f / t;
-  const int k = top_k[row];
-  const float p = top_p[row];
-  float thr = -INFINITY;
-  if ((k > 0 && k < V) || p < 1.f) {
-    float mx = -INFINITY, mn = INFINITY;
-#pragma unroll
-    for (int e = 0; e < NE; ++e) {
-      const float x = val(e);
+    R.each([&](float x, int) {
       mx = fmaxf(mx, x);
       if (x != -INFINITY) mn = fminf(mn, x);
-    }
+    });
     mx = block_max(mx, sv);
     mn = -block_max(-mn, sv);
-    if (k > 0 && k < V) {  // largest tau with count(z >= tau) >= k
-      float lo = mn, hi = mx;
-      for (int it = 0; it < 32; ++it) {
-        const float mid = 0.5f * (lo + hi);
-        float cnt = 0.f;
-        opaque();
-#pragma unroll
-        for (int e = 0; e < NE; ++e) cnt += val(e) >= mid ? 1.f : 0.f;
-        cnt = block_sum(cnt, sv);
-        if (cnt >= static_cast<float>(k)) lo = mid; else hi = mid;
+    if (mx == INFINITY) {  // nothing below an infinite logit has a share
+      thr = mx;
+    } else if (mx > -INFINITY) {
+      for (int by_share = 0; by_share < 2; ++by_share) {
+        if (by_share ? p < 1.f : k > 0 && k < V)
+          thr = fmaxf(thr, select_threshold(R, L, sv, by_share != 0, by_share ? static_cast<double>(p) : static_cast<double>(k),
+                                            mx, invt2, by_share ? fmaxf(mn, mx - 88.f * t) : mn, mx));
       }
-      thr = lo;
-    }
-    if (p < 1.f) {  // largest tau with mass(z >= tau) >= p * total, mass in softmax(z / T)
-      float tot = 0.f;
-#pragma unroll
-      for (int e = 0; e < NE; ++e) {
-        tot += __expf((val(e) - mx) * invt);
-        __builtin_amdgcn_sched_barrier(0);  // one element at a time: keeps the row in registers
-      }
-      tot = block_sum(tot, sv);
-      float lo = fmaxf(mn, mx - 88.f * t), hi = mx;
-      for (int it = 0; it < 32; ++it) {
-        const float mid = 0.5f * (lo + hi);
-        float mass = 0.f;
-        opaque();
-#pragma unroll
-        for (int e = 0; e < NE; ++e) {
-          const float x = val(e);
-          mass += x >= mid ? __expf((x - mx) * invt) : 0.f;
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        mass = block_sum(mass, sv);
-        if (mass >= p * tot) lo = mid; else hi = mid;
-      }
-      thr = fmaxf(thr, lo);
     }
   }
   const uint32_t key = hash_u32(static_cast<uint32_t>(static_cast<uint64_t>(seeds[row]) * 0x9E3779B1ull +
                                                       static_cast<uint64_t>(steps[row])));
-  const float invt2 = invt * kSLog2e;
   ArgMax a{-INFINITY, 0x7FFFFFFF};
-#pragma unroll
-  for (int e = 0; e < NE; ++e) {
-    const float x = val(e);
-    const int v = idx(e);
+  R.each([&](float x, int v) {
     if (v < V && x >= thr) a = better(a, ArgMax{x * invt2 + gumbel2(key, v), v});
-    if ((e & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // 4 independent hash/log chains in flight
-  }
-  ArgMax res = block_argmax(a, sv, si);
-  if (tid == 0) out[row] = res.i;
+  });
+  const ArgMax r = block_argmax(a, sv, si);
+  if (threadIdx.x == 0) out[row] = r.i;
 }
 
 void launch_sample(int64_t* out, const void* logits, bool bf16, int B, int V, long row_stride,
@@ -288,26 +338,22 @@ void launch_sample(int64_t* out, const void* logits, bool bf16, int B, int V, lo
                    const int64_t* steps, hipStream_t s) {
   if (B == 0) return;
   const bool vec = V % 8 == 0 && row_stride % 8 == 0 && (reinterpret_cast<uintptr_t>(logits) & 15) == 0;
-  static const bool reg_ok = [] {  // MXS_SAMPLE_REG=0: the memory form (A/B measurements)
-    const char* e = std::getenv("MXS_SAMPLE_REG");
-    return e == nullptr || e[0] != '0';
-  }();
-  if (reg_ok && bf16 && vec && V <= 2048 * 64) {
-    if (V <= 2048 * 16)
-      hipLaunchKernelGGL(sample_reg_kernel<16>, dim3(B), dim3(1024), 0, s, out, static_cast<const bf16_t*>(logits), V,
-                         row_stride, temperature, top_p, top_k, seeds, steps);
-    else
-      hipLaunchKernelGGL(sample_reg_kernel<64>, dim3(B), dim3(1024), 0, s, out, static_cast<const bf16_t*>(logits), V,
-                         row_stride, temperature, top_p, top_k, seeds, steps);
-    MXS_CHECK_LAUNCH();
-    return;
+  auto run = [&](auto kernel, auto* z) {
+    hipLaunchKernelGGL(kernel, dim3(B), dim3(1024), 0, s, out, z, V, row_stride, vec, temperature, top_p, top_k, seeds, steps);
+  };
+  // registers hold a row up to what 1024 threads of 128 VGPRs have room for: 160 bf16 or 64 fp32 logits a thread
+  if (bf16) {
+    const auto* z = static_cast<const bf16_t*>(logits);
+    if (vec && V <= 1024 * 32) run(sample_kernel<RegRow16<32>>, z);
+    else if (vec && V <= 1024 * 128) run(sample_kernel<RegRow16<128>>, z);
+    else if (vec && V <= 1024 * 160) run(sample_kernel<RegRow16<160>>, z);
+    else run(sample_kernel<MemRow<bf16_t>>, z);
+  } else {
+    const auto* z = static_cast<const float*>(logits);
+    if (vec && V <= 1024 * 32) run(sample_kernel<RegRow32<32>>, z);
+    else if (vec && V <= 1024 * 64) run(sample_kernel<RegRow32<64>>, z);
+    else run(sample_kernel<MemRow<float>>, z);
   }
-  if (bf16)
-    hipLaunchKernelGGL(sample_kernel<bf16_t>, dim3(B), dim3(1024), 0, s, out, static_cast<const bf16_t*>(logits), V,
-                       row_stride, temperature, top_p, top_k, seeds, steps);
-  else
-    hipLaunchKernelGGL(sample_kernel<float>, dim3(B), dim3(1024), 0, s, out, static_cast<const float*>(logits), V,
-                       row_stride, temperature, top_p, top_k, seeds, steps);
   MXS_CHECK_LAUNCH();
 }
 
