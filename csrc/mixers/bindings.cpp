@@ -1,5 +1,6 @@
 // torch bindings of the mixer kernels (mxserve/_M): shape and dtype checks on the host, so that a
 // launch never reads or writes outside what the kernels and their grids assume.
+#include "chunk_attention.h"
 #include "bind_util.h"
 #include "column_scan.h"
 #include "differential_attention.h"
@@ -603,6 +604,64 @@ bool latent_attention(at::Tensor out, at::Tensor q, at::Tensor cache, at::Tensor
       static_cast<int>(window), stream());
 }
 
+void latent_plan(at::Tensor base, at::Tensor offs, at::Tensor qsl, at::Tensor seq_lens, int64_t window) {
+  const int64_t S = seq_lens.numel();
+  TORCH_CHECK(window >= 0 && window < (1LL << 30), "window out of range");
+  mxs::launch_latent_plan(const_cast<int*>(i32(base, S, "base")), const_cast<int*>(i32(offs, S + 1, "offs")), i32(qsl, S + 1, "qsl"),
+                          i32(seq_lens, S, "seq_lens"), static_cast<int>(S), static_cast<int>(window), stream());
+}
+
+void latent_rows(at::Tensor out, at::Tensor cache, at::Tensor block_tables, at::Tensor base, at::Tensor offs, int64_t koff,
+                 int64_t bs) {
+  const int64_t n = out.size(0), dk = out.size(1), S = base.numel();
+  check_cache(cache, true, koff, koff, 1, dk, 0, bs);
+  TORCH_CHECK(bs == 16 && dk % 8 == 0 && koff % 8 == 0 && cache.stride(0) % 8 == 0 &&
+                  reinterpret_cast<uintptr_t>(cache.data_ptr()) % 16 == 0, "latent rows: whole 16-byte pieces in pages of 16");
+  TORCH_CHECK(out.is_cuda() && out.is_contiguous() && is_bf(out), "out: contiguous bf16 [n, dk]");
+  TORCH_CHECK(block_tables.is_cuda() && block_tables.scalar_type() == at::kInt && block_tables.dim() == 2 &&
+                  block_tables.size(0) >= S && block_tables.stride(1) == 1, "block_tables: int32 [S, max_blocks]");
+  mxs::launch_latent_rows((mxs::bf16_t*)out.data_ptr(), (const mxs::bf16_t*)cache.data_ptr(), cache.stride(0),
+                          block_tables.data_ptr<int>(), static_cast<int>(block_tables.stride(0)), i32(base, S, "base"),
+                          i32(offs, S + 1, "offs"), static_cast<int>(S), static_cast<int>(n), static_cast<int>(koff),
+                          static_cast<int>(dk), stream());
+}
+
+bool expanded_attention(at::Tensor out, at::Tensor q, at::Tensor kv, at::Tensor rows, at::Tensor base, at::Tensor qsl,
+                        at::Tensor seq_lens, int64_t H, int64_t dn, int64_t dr, int64_t dv, int64_t rank, double scale,
+                        int64_t max_query_len, OptT sink, int64_t window) {
+  const int64_t T = q.size(0), S = seq_lens.numel(), n = kv.size(0);
+  TORCH_CHECK(window >= 0 && window < (1LL << 30) && H >= 1 && dn >= 8 && dr >= 8 && dv >= 16, "head sizes out of range");
+  mxs::ChunkArgs a{};
+  a.q = (const mxs::bf16_t*)mat(q, true, T, H * (dn + dr), "q");
+  a.q_stride = q.stride(0);
+  a.kx = (const mxs::bf16_t*)mat(kv, true, n, H * (dn + dv), "kv");
+  a.x_stride = kv.stride(0);
+  a.vx = a.kx + H * dn;
+  a.kr = (const mxs::bf16_t*)mat(rows, true, n, rank + dr, "rows") + rank;
+  a.r_stride = rows.stride(0);
+  TORCH_CHECK(out.is_cuda() && out.is_contiguous() && out.dim() == 2 && out.size(0) == T && out.size(1) == H * dv && is_bf(out),
+              "out: contiguous bf16 [T, H*dv]");
+  if (T == 0 || S == 0 || n == 0) return T == 0;
+  if (dn % 8 || dr % 8 || rank % 8 || a.x_stride % 8 || a.r_stride % 8 || a.q_stride % 4 || a.x_stride >= (1LL << 26) ||
+      reinterpret_cast<uintptr_t>(a.kx) % 16 || reinterpret_cast<uintptr_t>(a.kr) % 16 || reinterpret_cast<uintptr_t>(a.q) % 8 ||
+      (H * dn) % 8)
+    return false;
+  a.out = (mxs::bf16_t*)out.data_ptr();
+  a.qsl = i32(qsl, S + 1, "qsl");
+  a.seq_lens = i32(seq_lens, S, "seq_lens");
+  a.base = i32(base, S, "base");
+  a.S = static_cast<int>(S);
+  a.H = a.G = static_cast<int>(H);
+  a.dk = static_cast<int>(dn + dr);
+  a.dn = static_cast<int>(dn);
+  a.dv = static_cast<int>(dv);
+  a.nrows = static_cast<int>(n);
+  a.scale = static_cast<float>(scale);
+  a.window = static_cast<int>(window);
+  a.sink = f32n(sink, H, "sink");
+  return mxs::launch_chunk_attention(a, static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(max_query_len, T))), stream());
+}
+
 void rope_half_into(at::Tensor out, at::Tensor x, at::Tensor positions, int64_t heads, int64_t x_dim, int64_t x_col,
                     int64_t out_dim, int64_t out_col, at::Tensor freqs, bool split_pairs, double mag) {
   const bool bf = is_bf(x);
@@ -829,6 +888,9 @@ PYBIND11_MODULE(_M, m) {
   m.def("gate_linear", &gate_linear);
   m.def("kv_write", &kv_write);
   m.def("window_attention", &window_attention);
+  m.def("latent_plan", &latent_plan);
+  m.def("latent_rows", &latent_rows);
+  m.def("expanded_attention", &expanded_attention);
   m.def("decay_scan", &decay_scan);
   m.def("mlstm_scan", &mlstm_scan);
   m.def("embed_scaled", &embed_scaled);

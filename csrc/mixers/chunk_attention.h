@@ -1,8 +1,10 @@
 // Softmax attention of prompt chunks on the matrix cores (chunk_attention.hip): what a launch needs.
 #pragma once
-#include "mix_common.h"
+#include <hip/hip_runtime.h>
 
 namespace mxs {
+
+typedef unsigned short bf16_t;  // raw bits
 
 struct ChunkArgs {
   bf16_t* out;  // [rows, H * dv]
@@ -19,14 +21,22 @@ struct ChunkArgs {
   long block_stride;
   const int* block_tables;
   int bt_stride, koff, voff;
-  // or in rows: key = kx[row * x_stride + head * 128 .. + 128) | kr[row * r_stride .. + dk - 128), value =
-  // vx[row * x_stride + head * dv ..], row = base[s] + key position
+  // or in rows (G = H): key = kx[row * x_stride + head * dn .. + dn) | kr[row * r_stride .. + dk - dn), value =
+  // vx[row * x_stride + head * dv ..], row = base[s] + key position, below nrows
   const bf16_t *kx, *vx, *kr;
   long x_stride, r_stride;
   const int* base;
+  int dn, nrows;
 };
 
 // false: head sizes that no kernel holds.  max_q: an upper bound of a sequence's rows in this launch.
 bool launch_chunk_attention(const ChunkArgs& a, int max_q, hipStream_t st);
+
+// base[s]: row of key position 0 of sequence s when the keys its chunk sees (with window > 0: from the page of the first
+// query's oldest one) lie back to back, offs[s]: its first row; offs[S]: rows in all.
+void launch_latent_plan(int* base, int* offs, const int* qsl, const int* seq_lens, int S, int window, hipStream_t st);
+// those rows of dk entries from pages of 16 at koff of a block, 16-byte pieces; at most n rows are written
+void launch_latent_rows(bf16_t* out, const bf16_t* cache, long block_stride, const int* block_tables, int bt_stride,
+                        const int* base, const int* offs, int S, int n, int koff, int dk, hipStream_t st);
 
 }  // namespace mxs

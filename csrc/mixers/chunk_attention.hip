@@ -14,8 +14,10 @@
 // exponentials, and 24 matrix instructions, and the two kinds hardly overlap (interleaving them by hand, four waves a SIMD,
 // walks paired long with short, and walks that begin at different keys all measured the same or slower).
 // 4,096 rows, 32 heads of 64 over 8 kv heads: 1,127 us with one wave per 16 rows of a head on the 16-wide instructions and
-// 2-byte reads of V (the form that this one replaced), 139 us; window 1,024: 75 us; 16 heads of 128: 192 us.
+// 2-byte reads of V (the form that this one replaced), 139 us; window 1,024: 75 us; 16 heads of 128: 192 us.  Keys of 128 + 64 and values of 128 expanded from latent rows of 576, 16 heads,
+// 4,096 rows: 217 us and 50 us for gathering and expanding, against 1,142 us over the rows themselves with folded queries.
 #include "chunk_attention.h"
+#include "mix_common.h"
 
 #include <algorithm>
 
@@ -78,12 +80,14 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
   const int kpr = dk >> 3, vpr = dv >> 3;  // pieces a row
   int krow[NK], vrow[NV], kat[NK], vat[NV];  // row inside the page (-1: none), place in LDS
   int kfrom[NK], vfrom[NV];                  // element offset from the page's base
+  bool kown[NK];                             // of a key in rows: the head's own part
 #pragma unroll
   for (int i = 0; i < NK; ++i) {
     const int idx = lane + 64 * (i * WPP + wv % WPP), r = idx / kpr, col = 8 * (idx - r * kpr);
     krow[i] = r < 16 ? r : -1;
     kat[i] = (wpage * 16 + r) * KROW + col;
-    kfrom[i] = PAGED ? 8 * idx : col < 128 ? r * static_cast<int>(a.x_stride) + col : r * static_cast<int>(a.r_stride) + col - 128;
+    kfrom[i] = PAGED ? 8 * idx : col < a.dn ? r * static_cast<int>(a.x_stride) + col : r * static_cast<int>(a.r_stride) + col - a.dn;
+    kown[i] = col < a.dn;
   }
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
@@ -106,6 +110,7 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
   const int* bt = PAGED ? a.block_tables + static_cast<long>(s) * a.bt_stride : nullptr;
   const int lastpage = PAGED ? min(glast >> 4, a.bt_stride - 1) : 0;
   const int dense0 = PAGED ? 0 : a.base[s];
+  const int kmax = PAGED ? glast : min(glast, a.nrows - 1 - dense0);  // the last key that may be read
   int page = 0;  // of the tile to be fetched next
   auto fetch_page = [&](int k0) {
     if constexpr (PAGED) page = bt[min((k0 >> 4) + wpage, lastpage)];
@@ -120,18 +125,18 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
       vb = blk + a.voff + g * 16 * dv;
     } else {
       const long r = dense0 + key0;
-      kb = a.kx + r * a.x_stride + g * 128;
+      kb = a.kx + r * a.x_stride + g * a.dn;
       vb = a.vx + r * a.x_stride + g * dv;
       rb = a.kr + r * a.r_stride;
     }
     // keys past the last one anybody here sees may hold anything: zeros
-    const int left = glast - key0;
+    const int left = kmax - key0;
 #pragma unroll
     for (int i = 0; i < NK; ++i) {
       kst[i] = make_uint4(0, 0, 0, 0);
       if (krow[i] >= 0 && krow[i] <= left) {
         const bf16_t* from = kb;
-        if constexpr (!PAGED) from = kat[i] - (wpage * 16 + krow[i]) * KROW < 128 ? kb : rb;
+        if constexpr (!PAGED) from = kown[i] ? kb : rb;
         kst[i] = *reinterpret_cast<const uint4*>(from + kfrom[i]);
       }
     }
@@ -284,13 +289,72 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
 
 bool launch_chunk_attention(const ChunkArgs& a, int max_q, hipStream_t st) {
   const bool paged = a.kx == nullptr;
-  if (a.dk % 16 || a.dv % 16 || a.dv > 128 || a.dk > (paged ? 128 : 192) || (!paged && (a.dk <= 128 || a.G != a.H))) return false;
+  if (a.dk % 16 || a.dv % 16 || a.dv > 128 || a.dk > (paged ? 128 : 192) || (!paged && (a.dn % 8 || a.dn > a.dk || a.G != a.H)))
+    return false;
   const dim3 grid(a.G, (static_cast<long>(max_q) * (a.H / a.G) + 127) / 128, a.S), block(256);
   if (!paged) hipLaunchKernelGGL((chunk_attention_kernel<192, 128, 32, false>), grid, block, 0, st, a);
   else if (a.dk <= 64 && a.dv <= 64) hipLaunchKernelGGL((chunk_attention_kernel<64, 64, 64, true>), grid, block, 0, st, a);
   else hipLaunchKernelGGL((chunk_attention_kernel<128, 128, 32, true>), grid, block, 0, st, a);
   MXS_CHECK_LAUNCH();
   return true;
+}
+
+// One workgroup: the sequences' row counts summed 256 at a time.
+__global__ void __launch_bounds__(256) latent_plan_kernel(int* __restrict__ base, int* __restrict__ offs,
+                                                          const int* __restrict__ qsl, const int* __restrict__ seq_lens,
+                                                          int S, int window) {
+  __shared__ int sum[256];
+  int before = 0;
+  for (int s0 = 0; s0 < S; s0 += 256) {
+    const int s = s0 + threadIdx.x;
+    int n = 0, firstkey = 0;
+    if (s < S) {
+      const int qlen = qsl[s + 1] - qsl[s], past = max(seq_lens[s] - qlen, 0);
+      firstkey = window > 0 ? max(past - window + 1, 0) & ~15 : 0;
+      n = qlen > 0 ? past + qlen - firstkey : 0;
+    }
+    sum[threadIdx.x] = n;
+    __syncthreads();
+    for (int o = 1; o < 256; o <<= 1) {
+      const int t = threadIdx.x >= o ? sum[threadIdx.x - o] : 0;
+      __syncthreads();
+      sum[threadIdx.x] += t;
+      __syncthreads();
+    }
+    if (s < S) {
+      offs[s] = before + sum[threadIdx.x] - n;
+      base[s] = offs[s] - firstkey;
+    }
+    before += sum[255];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) offs[S] = before;
+}
+
+void launch_latent_plan(int* base, int* offs, const int* qsl, const int* seq_lens, int S, int window, hipStream_t st) {
+  hipLaunchKernelGGL(latent_plan_kernel, dim3(1), dim3(256), 0, st, base, offs, qsl, seq_lens, S, window);
+  MXS_CHECK_LAUNCH();
+}
+
+__global__ void __launch_bounds__(256) latent_rows_kernel(uint4* __restrict__ out, const bf16_t* __restrict__ cache, long block_stride,
+                                                          const int* __restrict__ block_tables, int bt_stride,
+                                                          const int* __restrict__ base, const int* __restrict__ offs, int S,
+                                                          int n, int koff, int pieces) {
+  const long i = blockIdx.x * 256l + threadIdx.x;
+  const int row = static_cast<int>(i / pieces), piece = static_cast<int>(i - static_cast<long>(row) * pieces);
+  if (row >= min(n, offs[S])) return;
+  const int s = seq_of_row(offs, S, row), key = row - base[s];
+  const int page = block_tables[static_cast<long>(s) * bt_stride + min(key >> 4, bt_stride - 1)];
+  out[i] = *reinterpret_cast<const uint4*>(cache + page * block_stride + koff + ((key & 15) * pieces + piece) * 8);
+}
+
+void launch_latent_rows(bf16_t* out, const bf16_t* cache, long block_stride, const int* block_tables, int bt_stride,
+                        const int* base, const int* offs, int S, int n, int koff, int dk, hipStream_t st) {
+  if (n == 0) return;
+  const int pieces = dk / 8;
+  hipLaunchKernelGGL(latent_rows_kernel, dim3((static_cast<long>(n) * pieces + 255) / 256), dim3(256), 0, st,
+                     reinterpret_cast<uint4*>(out), cache, block_stride, block_tables, bt_stride, base, offs, S, n, koff, pieces);
+  MXS_CHECK_LAUNCH();
 }
 
 }  // namespace mxs

@@ -8,6 +8,7 @@
 // A sink (fp32 [H], optional) is one more key per head with the score sink[h], not scaled, and no
 // value: the running maximum starts at it and the running sum at 1 instead of -inf and 0.
 #include "chunk_attention.h"
+#include "mix_common.h"
 
 namespace mxs {
 

@@ -371,7 +371,7 @@ class ModelRunner:
         hist_init, self._hist_init = self._hist_init, []
         return dict(S=S, T=T, nd=nd, max_q=max_q, max_seq=max(lens), sample_rows=sample_rows, U=U,
                     big_update=big_update, graph_bs=graph_bs, lp=lp, pen=use_pen, hist_init=hist_init,
-                    n_score=n_score)
+                    n_score=n_score, chunks=tuple((s.start, s.num_new_tokens) for s in pre))
 
     def _upload(self, meta: dict) -> None:
         self.buf.upload()
@@ -595,7 +595,7 @@ class ModelRunner:
                           seq_lens=v["seq_lens"], query_start_loc=v["qsl"], logits_indices=v["logits_indices"],
                           num_decodes=nd, num_prefills=S - nd, num_prefill_tokens=T - nd,
                           max_query_len=meta["max_q"] or 1, max_seq_len=meta["max_seq"], prefill_query_start_loc=pq,
-                          sample_seq=v["sseq"], state_rows=v["rows"], state=self.state)
+                          sample_seq=v["sseq"], state_rows=v["rows"], state=self.state, chunks=meta.get("chunks"))
         inp = v["input_ids"]
         if nd:
             d_in = inp[:nd]

@@ -42,6 +42,8 @@ class AttnMetadata:
     # models with recurrent layers: each sequence's slot in the fp32 state pool [slots, state_floats]
     state_rows: Optional[torch.Tensor] = None  # [S] int32
     state: Optional[torch.Tensor] = None
+    # (cached tokens, new tokens) of every sequence behind the first num_decodes, known to the host; None: not said
+    chunks: Optional[tuple] = None
 
     @property
     def num_tokens(self) -> int:

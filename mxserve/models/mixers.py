@@ -73,6 +73,43 @@ class StepContext:
             t = self.tables[key] = seqmix.rotary_table(self.md.positions, freqs, mag)
         return t
 
+    def expansion(self, window: int) -> Optional[tuple]:
+        """(base, offs, rows): where the latent rows that this step's chunks see lie when they are gathered for every head to
+        expand its own keys and values from them; None when the chunks are too short for that to pay, or their lengths are
+        not known here."""
+        key = ("expansion", window)
+        if key not in self.tables:
+            self.tables[key] = self._plan_expansion(window)
+        return self.tables[key]
+
+    def _plan_expansion(self, window: int) -> Optional[tuple]:
+        md = self.md
+        chunks, nd = getattr(md, "chunks", None), getattr(md, "num_decodes", 0)
+        if not chunks or not md.seq_lens.is_cuda or len(chunks) + nd != md.seq_lens.numel():
+            return None
+        rows = pairs = 0
+        for past, n in chunks:
+            first = max(past - window + 1, 0) // 16 * 16 if window > 0 else 0
+            rows += past + n - first
+            pairs += n * min(past + (n + 1) // 2, window if window > 0 else 1 << 30)
+        if pairs < EXPAND_MIN_QUERIES * rows:
+            return None
+        return seqmix.latent_plan(self.chunk_rows(), md.seq_lens[nd:], window) + (rows,)
+
+    def chunk_rows(self) -> torch.Tensor:
+        """First rows of the sequences behind the single tokens, counted from the first of them."""
+        nd = getattr(self.md, "num_decodes", 0)
+        return self.md.prefill_query_start_loc if nd else self.md.query_start_loc
+
+
+# A latent attention's chunk expands keys and values per head where the gathered rows meet at least this many queries on
+# average.  Per head a key costs 2 * rank * (dim + vdim) operations to expand and every pair of a query and a key
+# 2 * (dim + rot_dim + vdim) instead of the folded form's 2 * (2 rank + rot_dim) (128 + 64, 128, rank 512: 262,144 against
+# 1,536 saved, so from 170 queries on by operations alone); the folded form runs them at a third of the rate as well.  4,096 new
+# tokens, 16 heads of these sizes: 1,142 + 50 us folded (attention, two batched products), 217 + 32 us expanded.
+EXPAND_MIN_QUERIES = 64
+EXPAND_MAX_BYTES = 1 << 30  # expanded keys and values of a layer; steps with more stay on the folded form
+
 
 class Mixer:
     kv_heads = dk = dv = 0  # paged K/V per token (0: none)
@@ -556,8 +593,10 @@ class LatentAttention(Mixer):
         self.freqs = self.freqs.to(w[p + "o"].device)
         if self.sink == "learned":
             _fp32(w, p + "sink")
-        # per-head factors of the two batched products: q'_plain = q_plain @ uk[h], out_h = latent_h @ uv[h]^T
-        w[p + "uk"] = w[p + "uk"].view(H, self.dn, self.rank).contiguous()
+        # both expansions as one projection of the latent, and per-head factors of the two batched products of the folded
+        # form: q'_plain = q_plain @ uk[h] (the projection's first rows as they are), out_h = latent_h @ uv[h]^T
+        w[p + "_ukv"] = torch.cat([w[p + "uk"], w[p + "uv"]]).contiguous()
+        w[p + "uk"] = w[p + "_ukv"][:H * self.dn].view(H, self.dn, self.rank)
         w[p + "uv"] = w[p + "uv"].view(H, self.vd, self.rank).transpose(1, 2).contiguous()
 
     def forward(self, parts: list, h: torch.Tensor, w: dict, ctx: StepContext, koff: int, voff: int, soff: int):
@@ -567,18 +606,51 @@ class LatentAttention(Mixer):
         cq = seqmix.latent_prep(dq, dkv, md.positions, md.slot_mapping, ctx.cache, koff, self.rank, ctx.block_size,
                                 self.freqs, w[p + "dq.norm"], w[p + "dkv.norm"], ctx.eps, self.split_pairs, self.mag)
         q = ops.linear(cq, w[p + "uq"])  # [T, H * (dn + dr)]
-        dq_, dk = self.dn + self.dr, self.dk
+        o = torch.empty(T, H * self.vd, dtype=q.dtype, device=q.device)
+        nd = T
+        if h.dtype == torch.bfloat16 and self._expand(q, o, w, ctx, koff):
+            nd = md.num_decodes
+        if nd:
+            self._fold(q[:nd], o[:nd], w, ctx, koff, nd < T)
+        return ops.linear(o, w[p + "o"])
+
+    def _expand(self, q: torch.Tensor, o: torch.Tensor, w: dict, ctx: StepContext, koff: int) -> bool:
+        """The rows behind the single tokens, every head on keys and values that it expands from the cached rows (as the
+        docstring's formulas read); False: they are too few, or of sizes that the kernel does not hold."""
+        md, p, H = ctx.md, self.p, self.heads
+        dq, nd = self.dn + self.dr, getattr(md, "num_decodes", 0)
+        plan = None
+        if dq <= 192 and dq % 16 == 0 and self.vd <= 128 and self.vd % 16 == 0 and self.dn % 8 == 0 and self.dr % 8 == 0 and \
+                self.rank % 8 == 0 and koff % 8 == 0 and ctx.cache.shape[1] % 8 == 0 and ctx.block_size == 16:
+            plan = ctx.expansion(self.window)
+        if plan is None or 2 * plan[2] * H * (self.dn + self.vd) > EXPAND_MAX_BYTES:
+            return False
+        base, offs, n = plan
+        rows = seqmix.latent_rows(ctx.cache, md.block_tables[nd:], base, offs, n, koff, self.dk, ctx.block_size)
+        kv = ops.linear(rows[:, :self.rank], w[p + "_ukv"])
+        qc = q[nd:]
+        seqmix.rope_half_into(qc, qc, md.positions[nd:], H, dq, self.dn, dq, self.dn, self.freqs, self.split_pairs, self.mag)
+        if seqmix.expanded_attention(qc, kv, rows, base, ctx.chunk_rows(), md.seq_lens[nd:], H, self.dn, self.dr, self.vd,
+                                     self.scale, md.max_query_len, w.get(p + "sink"), self.window, o[nd:]) is None:
+            raise RuntimeError(f"{p}: no kernel for heads of {self.dn} + {self.dr} / {self.vd} entries")  # q is turned already
+        return True
+
+    def _fold(self, q: torch.Tensor, o: torch.Tensor, w: dict, ctx: StepContext, koff: int, singles: bool) -> None:
+        """Every row (or, with `singles`, the step's single tokens) over the cached rows themselves, W_uk folded into the
+        query and W_uv applied to the weighted sum."""
+        md, p, H = ctx.md, self.p, self.heads
+        T, dq_, dk = q.shape[0], self.dn + self.dr, self.dk
+        bt, qsl, lens, mq = md.block_tables, md.query_start_loc, md.seq_lens, md.max_query_len
+        if singles:
+            bt, qsl, lens, mq = bt[:T], qsl[:T + 1], lens[:T], 1
         qf = torch.empty(T, H * dk, dtype=q.dtype, device=q.device)
         # the plain part through W_uk^T, head by head, straight into its columns of the folded query
         torch.bmm(q.view(T, H, dq_)[:, :, :self.dn].transpose(0, 1), w[p + "uk"],
                   out=qf.view(T, H, dk)[:, :, :self.rank].transpose(0, 1))
-        seqmix.rope_half_into(qf, q, md.positions, H, dq_, self.dn, dk, self.rank, self.freqs, self.split_pairs, self.mag)
-        lat = seqmix.latent_attention(qf, ctx.cache, md.block_tables, md.query_start_loc, md.seq_lens, koff, H, dk,
-                                      self.rank, ctx.block_size, self.scale, md.max_query_len,
+        seqmix.rope_half_into(qf, q, md.positions[:T], H, dq_, self.dn, dk, self.rank, self.freqs, self.split_pairs, self.mag)
+        lat = seqmix.latent_attention(qf, ctx.cache, bt, qsl, lens, koff, H, dk, self.rank, ctx.block_size, self.scale, mq,
                                       getattr(md, "max_seq_len", 0), sink=w.get(p + "sink"), window=self.window)
-        o = torch.empty(T, H * self.vd, dtype=q.dtype, device=q.device)
         torch.bmm(lat.view(T, H, self.rank).transpose(0, 1), w[p + "uv"], out=o.view(T, H, self.vd).transpose(0, 1))
-        return ops.linear(o, w[p + "o"])
 
 
 class TalkingAttention(Mixer):

@@ -1196,6 +1196,74 @@ def latent_attention(q: torch.Tensor, cache: torch.Tensor, block_tables: torch.T
                             int(window), 0, max_query_len, sink=sink, v_stride=dk)
 
 
+def latent_plan(qsl: torch.Tensor, seq_lens: torch.Tensor, window: int = 0) -> tuple:
+    """Where the cached rows that a step's chunks see lie when they are gathered back to back (latent_rows): (base int32 [S],
+    the row of a sequence's key position 0, and offs int32 [S + 1], its first row).  With window > 0 a sequence's rows begin
+    at the page of its first query's oldest visible key."""
+    S = seq_lens.numel()
+    base = torch.empty(S, dtype=torch.int32, device=seq_lens.device)
+    offs = torch.empty(S + 1, dtype=torch.int32, device=seq_lens.device)
+    if _gpu(seq_lens):
+        ext().latent_plan(base, offs, qsl, seq_lens, int(window))
+        return base, offs
+    qlen = qsl[1:S + 1] - qsl[:S]
+    past = (seq_lens - qlen).clamp(min=0)
+    first = (past - window + 1).clamp(min=0) // 16 * 16 if window > 0 else torch.zeros_like(past)
+    offs[0] = 0
+    offs[1:] = torch.where(qlen > 0, past + qlen - first, torch.zeros_like(past)).cumsum(0)
+    base.copy_(offs[:S] - first)
+    return base, offs
+
+
+def latent_rows(cache: torch.Tensor, block_tables: torch.Tensor, base: torch.Tensor, offs: torch.Tensor, n: int, koff: int,
+                dk: int, block_size: int) -> torch.Tensor:
+    """The cached rows [n, dk] of latent_plan's places; n = offs[S], known to the host."""
+    out = torch.empty(n, dk, dtype=cache.dtype, device=cache.device)
+    if _gpu(cache):
+        ext().latent_rows(out, cache, block_tables, base, offs, int(koff), int(block_size))
+        return out
+    kc = cache[:, koff:koff + block_size * dk].view(-1, block_size, dk)
+    for s in range(base.numel()):
+        a, e = int(offs[s]), int(offs[s + 1])
+        key = torch.arange(a, e) - int(base[s])
+        out[a:e] = kc[block_tables[s].long()[key // block_size], key % block_size]
+    return out
+
+
+def expanded_attention(q: torch.Tensor, kv: torch.Tensor, rows: torch.Tensor, base: torch.Tensor, qsl: torch.Tensor,
+                       seq_lens: torch.Tensor, num_heads: int, dn: int, dr: int, dv: int, scale: float, max_query_len: int,
+                       sink: Optional[torch.Tensor] = None, window: int = 0,
+                       out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """Causal softmax attention of chunks over keys and values that every head expanded from gathered latent rows.
+    q [T, H*(dn + dr)], kv [n, H*dn + H*dv]: the heads' plain key parts, then their values; the last dr entries of `rows`
+    [n, rank + dr] are the key part that all heads share.  Row of key position j of sequence s: base[s] + j.  sink, window
+    as in latent_attention.  -> [T, H*dv] (in `out` if given); None: head sizes that the kernel does not hold."""
+    T, H, rank = q.shape[0], num_heads, rows.shape[1] - dr
+    if out is None:
+        out = torch.empty(T, H * dv, dtype=q.dtype, device=q.device)
+    if _gpu(q):
+        ok = q.dtype == torch.bfloat16 and ext().expanded_attention(out, q, kv, rows, base, qsl, seq_lens, H, dn, dr, dv, rank,
+                                                                    float(scale), int(max_query_len), sink, int(window))
+        return out if ok else None
+    ql, sl, bl = qsl.tolist(), seq_lens.tolist(), base.tolist()
+    for s in range(len(sl)):
+        a, e = ql[s], ql[s + 1]
+        if e <= a:
+            continue
+        lo = max(0, -bl[s])
+        r = torch.arange(lo, sl[s]) + bl[s]
+        K = torch.cat([kv[r, :H * dn].view(-1, H, dn), rows[r, rank:].unsqueeze(1).expand(-1, H, -1)], -1).float()
+        sc = torch.einsum("mhd,nhd->hmn", q[a:e].reshape(e - a, H, dn + dr).float(), K) * scale
+        i, j = torch.arange(sl[s] - (e - a), sl[s]).unsqueeze(1), torch.arange(lo, sl[s]).unsqueeze(0)
+        seen = (j <= i) & (i - j < window) if window > 0 else j <= i
+        sc = sc.masked_fill(~seen.unsqueeze(0), float("-inf"))
+        if sink is not None:
+            sc = torch.cat([sc, sink.float().view(-1, 1, 1).expand(-1, sc.shape[1], 1)], dim=-1)
+        p = torch.softmax(sc, dim=-1)[..., :r.numel()]
+        out[a:e] = torch.einsum("hmn,nhd->mhd", p, kv[r, H * dn:].view(-1, H, dv).float()).reshape(e - a, -1).to(out.dtype)
+    return out
+
+
 # ----------------------------------------------------------------------------- routed experts
 def route_topk(logits: torch.Tensor, k: int, renorm: bool = False, softmax: bool = False, *,
                correction: Optional[torch.Tensor] = None, groups: int = 1, keep: int = 1, scale: float = 1.0) -> tuple:
