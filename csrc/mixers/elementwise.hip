@@ -55,11 +55,6 @@ __global__ void __launch_bounds__(256) resid_update_kernel(float* __restrict__ x
 // update to the norm, so that every operand is read once, 16 bytes at a time, all of a row's loads ahead of the first
 // sum.  4,096 rows of 2,048: 34 -> 20 us (20 us are its bytes); 64 rows, as in a decode step: 11.7 -> 4.0 us (launch and
 // two or three block sums).
-__device__ __forceinline__ void ld8f(const bf16_t* p, float* o) { load16(p, o); }
-__device__ __forceinline__ void ld8f(const float* p, float* o) { load16(p, o); load16(p + 4, o + 4); }
-__device__ __forceinline__ void st8f(bf16_t* p, const float* o) { store16(p, o); }
-__device__ __forceinline__ void st8f(float* p, const float* o) { store16(p, o); store16(p + 4, o + 4); }
-
 template <typename T, int NP>
 __global__ void __launch_bounds__(256) resid_update_rows_kernel(
     float* __restrict__ x, const T* __restrict__ a, long a_stride, const T* __restrict__ wa, const T* __restrict__ b,

@@ -62,6 +62,12 @@ __device__ __forceinline__ void store16(float* p, const float* v) {
   *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
 }
 
+// 8 neighbouring elements
+__device__ __forceinline__ void ld8f(const bf16_t* p, float* o) { load16(p, o); }
+__device__ __forceinline__ void ld8f(const float* p, float* o) { load16(p, o); load16(p + 4, o + 4); }
+__device__ __forceinline__ void st8f(bf16_t* p, const float* o) { store16(p, o); }
+__device__ __forceinline__ void st8f(float* p, const float* o) { store16(p, o); store16(p + 4, o + 4); }
+
 __device__ __forceinline__ float silu_f(float z) { return z / (1.f + expf(-z)); }
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.f / (1.f + expf(-z)); }
 __device__ __forceinline__ float logsigmoid_f(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }

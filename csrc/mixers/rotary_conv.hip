@@ -3,6 +3,8 @@
 // cache write in one launch, turning attention outputs back, the convolution with its carried
 // inputs (alone, or with the query factor and the page write), and the norm of a recurrent mixer's read-out with its gate.  Activations and weights are
 // bf16 or fp32; angles, norms, sums and activations are fp32 with one rounding at the store.
+#include <algorithm>
+
 #include "mix_common.h"
 
 namespace mxs {
@@ -109,6 +111,102 @@ __global__ void __launch_bounds__(64) rope_rows_kernel(T* __restrict__ out, long
   }
 }
 
+// The same two for heads of whole, aligned pieces of 8 (key heads of 8 times a power of two, so that a norm is a sum over
+// neighbouring lanes): a workgroup per token, which makes the token's turns once in LDS for all heads.  A wave per token
+// and head turned 32 pairs on 2-byte accesses and made its sines itself.  4,096 tokens, 32 + 8 + 8 heads of 64 with
+// norms: 54 -> 15.4 us; turning 32 heads back: 31 -> 8.2 us (10 and 7 us are their bytes).
+template <typename T>
+__device__ __forceinline__ void turn8(float* x, const float2* cs, int d, int nf) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int pr = d / 2 + i;
+    if (pr < nf) {
+      const float2 t = cs[pr];
+      const float a = x[2 * i], b = x[2 * i + 1];
+      x[2 * i] = a * t.x - b * t.y;
+      x[2 * i + 1] = b * t.x + a * t.y;
+    }
+  }
+}
+__device__ __forceinline__ void make_turns(float2* cs, const float* freqs, int nf, float pos) {
+  for (int i = threadIdx.x; i < nf; i += blockDim.x) {
+    float sn, c;
+    sincosf(pos * freqs[i], &sn, &c);
+    cs[i] = make_float2(c, sn);
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(512) rope_qkv_cache_wide_kernel(
+    T* __restrict__ q, long q_stride, const T* __restrict__ k, long k_stride, const T* __restrict__ v, long v_stride,
+    const int64_t* __restrict__ positions, const int64_t* __restrict__ slots, T* __restrict__ cache, long block_stride,
+    int koff, int voff, int H, int G, int dk, int dv, int bs, const float* __restrict__ freqs, int nf,
+    const T* __restrict__ q_norm, const T* __restrict__ k_norm, float eps, const float* __restrict__ v_freqs, int nvf) {
+  extern __shared__ float2 cs[];  // [nf] then [nvf]
+  const long t = blockIdx.x;
+  const int LP = dk / 8, nq = H * LP, nk = k ? G * LP : 0, n = nq + nk + (k ? G * dv / 8 : 0);
+  int i = threadIdx.x;
+  float x[8];
+  auto fetch = [&] {
+    if (i < n) ld8f(i < nq ? q + t * q_stride + 8 * i : i < nq + nk ? k + t * k_stride + 8 * (i - nq) : v + t * v_stride + 8 * (i - nq - nk), x);
+  };
+  fetch();  // under way while the turns are made
+  const int64_t slot = k ? slots[t] : -1;
+  const float pos = static_cast<float>(positions[t]);
+  make_turns(cs, freqs, nf, pos);
+  make_turns(cs + nf, v_freqs, nvf, pos);
+  __syncthreads();
+  T* page = cache + (slot < 0 ? 0 : slot / bs) * block_stride;
+  const int off = static_cast<int>(slot < 0 ? 0 : slot % bs);
+  for (; i < n; i += blockDim.x, fetch()) {
+    if (i < nq + nk) {
+      const bool isq = i < nq;
+      const int j = isq ? i : i - nq, d = 8 * (j % LP), head = j / LP;
+      const T* nw = isq ? q_norm : k_norm;
+      if (nw) {
+        float s = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += x[e] * x[e];
+        for (int o = 1; o < LP; o <<= 1) s += __shfl_xor(s, o, 64);
+        const float inv = rsqrtf(s / static_cast<float>(dk) + eps);
+        float w[8];
+        ld8f(nw + d, w);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = x[e] * inv * w[e];
+      }
+      turn8<T>(x, cs, d, nf);
+      if (isq) st8f(q + t * q_stride + 8 * j, x);
+      else if (slot >= 0) st8f(page + koff + (static_cast<long>(head) * bs + off) * dk + d, x);
+    } else if (slot >= 0) {
+      const int c = 8 * (i - nq - nk), g = c / dv, d = c - g * dv;
+      turn8<T>(x, cs + nf, d, nvf);
+      st8f(page + voff + (static_cast<long>(g) * bs + off) * dv + d, x);
+    }
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) rope_rows_wide_kernel(T* __restrict__ out, long out_stride, const T* __restrict__ x,
+                                                             long x_stride, const int64_t* __restrict__ positions, int heads,
+                                                             int dim, const float* __restrict__ freqs, int nf, float sign,
+                                                             float scale) {
+  extern __shared__ float2 cs[];
+  const long t = blockIdx.x;
+  const int n = heads * dim / 8;
+  int i = threadIdx.x;
+  float v[8];
+  if (i < n) ld8f(x + t * x_stride + 8 * i, v);
+  make_turns(cs, freqs, nf, static_cast<float>(positions[t]) * sign);
+  __syncthreads();
+  while (i < n) {
+    turn8<T>(v, cs, 8 * i % dim, nf);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] *= scale;
+    st8f(out + t * out_stride + 8 * i, v);
+    if ((i += blockDim.x) < n) ld8f(x + t * x_stride + 8 * i, v);
+  }
+}
+
 // y[t, c] = act(bias[c] + sum_j w[j, c] x[t - (taps-1) + j, c]), w tap-major [taps, C]; inputs before the
 // chunk come from the sequence's state rows [taps-1, C] (oldest first), zeros for a sequence's first
 // tokens.  A thread takes V consecutive channels: V = 16 bytes' worth when rows, weights and channel
@@ -192,6 +290,85 @@ __global__ void __launch_bounds__(256) causal_conv_kernel(T* __restrict__ out, c
   }
   if constexpr (WIDE) store_piece(out + static_cast<long>(t) * C + c, acc);
   else stf(out + static_cast<long>(t) * C + c, acc[0]);
+}
+
+// The wide form for chunks: a thread takes its channels of 4 consecutive rows, so that a row is read once and not once per
+// tap; what a row's filter reaches back to is carried from row to row, and taken anew where a sequence begins.  The terms
+// of a sum are those of the kernel above, in its order.  4,096 rows of 6,144 channels, 4 taps: 48 -> 37 us.
+constexpr int kConvRows = 4;
+template <typename T, int TAPS>
+__global__ void __launch_bounds__(256) causal_conv_rows_kernel(T* __restrict__ out, const T* __restrict__ x, long x_stride,
+                                                               const T* __restrict__ w, const T* __restrict__ bias,
+                                                               const float* __restrict__ state, long state_stride,
+                                                               const int* __restrict__ state_rows, long off,
+                                                               const int* __restrict__ qsl, const int* __restrict__ seq_lens,
+                                                               int S, int rows, int C, int silu) {
+  constexpr int V = Piece<T>::N;
+  const int t0 = blockIdx.x * kConvRows;
+  const int c = (blockIdx.y * 256 + threadIdx.x) * V;
+  if (c >= C) return;
+  uint4 raw[kConvRows];
+#pragma unroll
+  for (int r = 0; r < kConvRows; ++r)
+    raw[r] = *reinterpret_cast<const uint4*>(x + static_cast<long>(min(t0 + r, rows - 1)) * x_stride + c);
+  float wv[TAPS][V], bv[V], hist[TAPS - 1][V];
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) load_piece(w + static_cast<long>(j) * C + c, wv[j]);
+#pragma unroll
+  for (int e = 0; e < V; ++e) bv[e] = 0.f;
+  if (bias) load_piece(bias + c, bv);
+  int s = seq_of_row(qsl, S, t0);
+  auto look_back = [&](int t) {  // the TAPS - 1 inputs before row t of sequence s
+    const int row0 = qsl[s], i = t - row0;
+    const bool fresh = seq_lens[s] - (qsl[s + 1] - row0) <= 0;
+#pragma unroll
+    for (int j = 0; j < TAPS - 1; ++j) {
+      const int src = i - (TAPS - 1) + j;
+      if (src >= 0) {
+        load_piece(x + static_cast<long>(row0 + src) * x_stride + c, hist[j]);
+      } else if (fresh) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) hist[j][e] = 0.f;
+      } else {
+        const float* sp = state + static_cast<long>(state_rows[s]) * state_stride + off + static_cast<long>(TAPS - 1 + src) * C + c;
+#pragma unroll
+        for (int e = 0; e < V; e += 4) load_piece(sp + e, hist[j] + e);
+      }
+    }
+  };
+  look_back(t0);
+#pragma unroll
+  for (int r = 0; r < kConvRows; ++r) {
+    const int t = t0 + r;
+    if (t >= rows) break;
+    if (r > 0 && t == qsl[s + 1]) {
+      do ++s; while (s + 1 < S && qsl[s + 1] <= t);
+      look_back(t);
+    }
+    float xv[V], acc[V];
+    if constexpr (V == 8) {
+      xv[0] = bf2f_lo(raw[r].x); xv[1] = bf2f_hi(raw[r].x); xv[2] = bf2f_lo(raw[r].y); xv[3] = bf2f_hi(raw[r].y);
+      xv[4] = bf2f_lo(raw[r].z); xv[5] = bf2f_hi(raw[r].z); xv[6] = bf2f_lo(raw[r].w); xv[7] = bf2f_hi(raw[r].w);
+    } else {
+      xv[0] = __uint_as_float(raw[r].x); xv[1] = __uint_as_float(raw[r].y);
+      xv[2] = __uint_as_float(raw[r].z); xv[3] = __uint_as_float(raw[r].w);
+    }
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+      acc[e] = bv[e];
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j) acc[e] += wv[j][e] * hist[j][e];
+      acc[e] += wv[TAPS - 1][e] * xv[e];
+      if (silu) acc[e] = silu_f(acc[e]);
+    }
+    store_piece(out + static_cast<long>(t) * C + c, acc);
+#pragma unroll
+    for (int j = 0; j + 1 < TAPS - 1; ++j)
+#pragma unroll
+      for (int e = 0; e < V; ++e) hist[j][e] = hist[j + 1][e];
+#pragma unroll
+    for (int e = 0; e < V; ++e) hist[TAPS - 2][e] = xv[e];
+  }
 }
 
 // The convolution without activation, from the fused projection to what attention reads: u = x + bias, the
@@ -345,6 +522,48 @@ __global__ void __launch_bounds__(256) gated_norm_kernel(T* __restrict__ out, lo
   }
 }
 
+// The same for slices of 8 LP NP entries, LP a power of two up to 64: LP neighbouring lanes hold a slice, 8 entries a lane and
+// step of LP lanes, from the activation to the store; a wave serves 64 / LP slices at once.  4,096 rows of 4,096, 8
+// slices, SiLU first: 48.6 -> 28 us; 64 rows: 11.2 -> 4.5 us.
+template <typename T, int NP>
+__global__ void __launch_bounds__(256) gated_norm_wide_kernel(T* __restrict__ out, long out_stride, const float* __restrict__ o,
+                                                              const T* __restrict__ gate, long g_stride,
+                                                              const T* __restrict__ w, int wn, int N, int n, int LP, float eps,
+                                                              int silu, int gate_first, float scale) {
+  const long row = blockIdx.x;
+  const int l = threadIdx.x & (LP - 1);  // LP divides 64
+  for (int sl = threadIdx.x / LP; sl * n < N; sl += 256 / LP) {
+    float v[NP][8], g[NP][8];
+    float s = 0.f;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const int c = sl * n + 8 * (l + p * LP);
+      ld8f(o + row * N + c, v[p]);
+      ld8f(gate + row * g_stride + c, g[p]);
+    }
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float a = silu ? silu_f(g[p][e]) : sigmoid_f(g[p][e]);
+        if (gate_first) v[p][e] *= a;
+        s += v[p][e] * v[p][e];
+        g[p][e] = gate_first ? 1.f : a;
+      }
+    for (int d = 1; d < LP; d <<= 1) s += __shfl_xor(s, d, 64);
+    const float inv = rsqrtf(s / static_cast<float>(n) + eps);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const int c = sl * n + 8 * (l + p * LP);
+      float wv[8];
+      ld8f(w + c % wn, wv);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) wv[e] = v[p][e] * inv * wv[e] * g[p][e] * scale;
+      st8f(out + row * out_stride + c, wv);
+    }
+  }
+}
+
 #define MIX_DISPATCH(bf, ...)                      \
   do {                                             \
     if (bf) { using T = bf16_t; __VA_ARGS__; }     \
@@ -365,6 +584,22 @@ void launch_rope_qkv_cache(void* q, long q_stride, const void* k, long k_stride,
                            const void* q_norm, const void* k_norm, float eps, const float* v_freqs, int nvf, bool bf,
                            hipStream_t st) {
   if (rows == 0) return;
+  auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  const int LP = dk / 8;
+  if (dk % 8 == 0 && LP <= 64 && (LP & (LP - 1)) == 0 && q_stride % 8 == 0 && al(q) && al(q_norm) && al(k_norm) &&
+      nf + nvf <= 4096 &&
+      (k == nullptr || (dv % 8 == 0 && k_stride % 8 == 0 && v_stride % 8 == 0 && al(k) && al(v) && al(cache) && koff % 8 == 0 &&
+                        voff % 8 == 0 && block_stride % 8 == 0))) {
+    // few tokens: a lane for every piece (64 tokens 3.8 us, 4.6 with 256 lanes); many: smaller workgroups pack better (4,096
+    // tokens 15.4 us, 18.3 with 512)
+    const int threads = std::min(rows <= 1024 ? 512 : 256, (H * LP + (k ? G * (LP + dv / 8) : 0) + 63) / 64 * 64);
+    MIX_DISPATCH(bf, hipLaunchKernelGGL(rope_qkv_cache_wide_kernel<T>, dim3(rows), dim3(threads), (nf + nvf) * sizeof(float2), st,
+                                        (T*)q, q_stride, (const T*)k, k_stride, (const T*)v, v_stride, positions, slots,
+                                        (T*)cache, block_stride, koff, voff, H, G, dk, dv, bs, freqs, nf, (const T*)q_norm,
+                                        (const T*)k_norm, eps, v_freqs, nvf));
+    MXS_CHECK_LAUNCH();
+    return;
+  }
   const dim3 grid(rows, H + (k != nullptr ? 2 * G : 0));
   MIX_DISPATCH(bf, hipLaunchKernelGGL(rope_qkv_cache_kernel<T>, grid, dim3(64), 0, st, (T*)q, q_stride, (const T*)k,
                                       k_stride, (const T*)v, v_stride, positions, slots, (T*)cache, block_stride, koff,
@@ -376,6 +611,13 @@ void launch_rope_qkv_cache(void* q, long q_stride, const void* k, long k_stride,
 void launch_rope_rows(void* out, long out_stride, const void* x, long x_stride, const int64_t* positions, int rows,
                       int heads, int dim, const float* freqs, int nf, float sign, float scale, bool bf, hipStream_t st) {
   if (rows == 0) return;
+  auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  if (dim % 8 == 0 && x_stride % 8 == 0 && out_stride % 8 == 0 && al(x) && al(out) && nf <= 4096) {
+    MIX_DISPATCH(bf, hipLaunchKernelGGL(rope_rows_wide_kernel<T>, dim3(rows), dim3(std::min(256, (heads * dim / 8 + 63) / 64 * 64)), nf * sizeof(float2), st, (T*)out, out_stride,
+                                        (const T*)x, x_stride, positions, heads, dim, freqs, nf, sign, scale));
+    MXS_CHECK_LAUNCH();
+    return;
+  }
   MIX_DISPATCH(bf, hipLaunchKernelGGL(rope_rows_kernel<T>, dim3(rows, heads), dim3(64), 0, st, (T*)out, out_stride,
                                       (const T*)x, x_stride, positions, dim, freqs, nf, sign, scale));
   MXS_CHECK_LAUNCH();
@@ -391,7 +633,17 @@ void launch_causal_conv(void* out, const void* x, long x_stride, const void* w, 
   auto al = [](const void* ptr) { return reinterpret_cast<uintptr_t>(ptr) % 16 == 0; };
   const bool wide = C % v == 0 && x_stride % v == 0 && al(x) && al(w) && al(out) && (bias == nullptr || al(bias)) &&
                     al(state) && state_stride % 4 == 0 && off % 4 == 0;
-  if (wide) {
+  if (wide && !single && taps >= 2 && taps <= 4) {
+    const dim3 grid((rows + kConvRows - 1) / kConvRows, (C / v + 255) / 256);
+#define MIX_CONV(TAPS)                                                                                                    \
+  MIX_DISPATCH(bf, hipLaunchKernelGGL((causal_conv_rows_kernel<T, TAPS>), grid, dim3(256), 0, st, (T*)out, (const T*)x,   \
+                                      x_stride, (const T*)w, (const T*)bias, state, state_stride, state_rows, off, qsl,  \
+                                      seq_lens, S, rows, C, silu))
+    if (taps == 2) MIX_CONV(2);
+    else if (taps == 3) MIX_CONV(3);
+    else MIX_CONV(4);
+#undef MIX_CONV
+  } else if (wide) {
     const int cw = (C / v + 255) / 256;
     MIX_DISPATCH(bf, hipLaunchKernelGGL((causal_conv_kernel<T, true>), dim3(rows, cw), dim3(256), 0, st, (T*)out,
                                         (const T*)x, x_stride, (const T*)w, (const T*)bias, state, state_stride,
@@ -444,6 +696,21 @@ void launch_gated_norm(void* out, long out_stride, const float* o, const void* g
                        int rows, int N, int groups, float eps, int silu, int gate_first, float scale, bool bf,
                        hipStream_t st) {
   if (rows == 0) return;
+  auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  const int n = N / groups, LP = n % 8 == 0 ? std::min(64, n / 8) : 0, np = LP ? n / 8 / LP : 0;
+  if (LP && (LP & (LP - 1)) == 0 && 8 * LP * np == n && (np == 1 || np == 2 || np == 4 || np == 8) && wn % 8 == 0 && N % 8 == 0 &&
+      g_stride % 8 == 0 && out_stride % 8 == 0 && al(out) && al(o) && al(gate) && al(w)) {
+#define MIX_GN(NP)                                                                                                     \
+  MIX_DISPATCH(bf, hipLaunchKernelGGL((gated_norm_wide_kernel<T, NP>), dim3(rows), dim3(256), 0, st, (T*)out, out_stride, o, \
+                                      (const T*)gate, g_stride, (const T*)w, wn, N, n, LP, eps, silu, gate_first, scale))
+    if (np == 1) MIX_GN(1);
+    else if (np == 2) MIX_GN(2);
+    else if (np == 4) MIX_GN(4);
+    else MIX_GN(8);
+#undef MIX_GN
+    MXS_CHECK_LAUNCH();
+    return;
+  }
   MIX_DISPATCH(bf, hipLaunchKernelGGL(gated_norm_kernel<T>, dim3(rows), dim3(256), 0, st, (T*)out, out_stride, o,
                                       (const T*)gate, g_stride, (const T*)w, wn, N, groups, eps, silu, gate_first, scale));
   MXS_CHECK_LAUNCH();

@@ -40,3 +40,65 @@ def test_softcap_rows(gpu, dt, T, V, pad):
     x = (20 * torch.randn(T, V + pad, generator=torch.Generator().manual_seed(V))).to(dt)[:, pad:]
     for cap in (0.0, 12.5):
         torch.testing.assert_close(seqmix.softcap(x.to(gpu), cap).cpu(), seqmix.softcap(x, cap), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("H,G,dk,dv,nf,nvf", [(4, 2, 8, 8, 2, 0), (6, 3, 16, 24, 8, 12), (32, 8, 64, 64, 32, 0), (5, 5, 64, 40, 9, 20),
+                                              (2, 1, 512, 16, 256, 8), (3, 1, 24, 16, 12, 0), (2, 2, 1024, 8, 4, 4)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_rotary_rows(gpu, dt, H, G, dk, dv, nf, nvf, norm):
+    g = torch.Generator().manual_seed(H * dk + nf)
+    T, bs, koff = 5, 16, 16
+    voff = koff + G * bs * dk
+    qkv = torch.randn(T, H * dk + G * (dk + dv), generator=g).to(dt)
+    cache = torch.randn(3, voff + G * bs * dv + 8, generator=g).to(dt)
+    pos, slots = torch.tensor([0, 7, 1000, 33, 5]), torch.tensor([40, 3, -1, 17, 0])
+    fr, vf = torch.rand(nf, generator=g), torch.rand(nvf, generator=g) if nvf else None
+    qn, kn = ((torch.randn(dk, generator=g)).to(dt) if norm else None for _ in range(2))
+    res = {}
+    for dev in ("cpu", gpu):
+        x, c = qkv.clone().to(dev), cache.clone().to(dev)
+        on = lambda t: None if t is None else t.to(dev)  # noqa: E731
+        q, k, v = x.split([H * dk, G * dk, G * dv], dim=1)
+        seqmix.rope_qkv_cache(q, k, v, on(pos), on(slots), c, koff, voff, H, G, dk, dv, bs, on(fr), on(qn), on(kn), 1e-5, on(vf))
+        y = torch.zeros(T, H * dk + 8, dtype=dt, device=dev)
+        seqmix.rope_rows(q, on(pos), H, dk, on(fr), -1.0, 0.7, y[:, 8:])
+        res[str(dev)] = (x.cpu(), c.cpu(), y.cpu())
+    for a, b in zip(*res.values()):
+        # angles of up to 1,000 turned in fp32: 2^-24 * 1000 of a turn either way
+        torch.testing.assert_close(a.float(), b.float(), **(dict(rtol=1e-4, atol=4e-4) if dt == torch.float32 else dict(rtol=2.0 ** -6, atol=2.0 ** -6)))
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("C", [8, 72, 2056])
+@pytest.mark.parametrize("taps", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("lens", [[1], [8], [9], [1, 1, 1, 1, 1, 1, 1, 1, 1], [3, 4, 1, 2, 17], [7, 1, 8, 16]])
+def test_convolution_rows(gpu, dt, C, taps, lens):
+    g = torch.Generator().manual_seed(C + taps + len(lens))
+    T, S = sum(lens), len(lens)
+    x = torch.randn(T, C + 16, generator=g).to(dt)[:, 16:]
+    w, b = torch.randn(taps, C, generator=g).to(dt), torch.randn(C, generator=g).to(dt)
+    state = torch.randn(S + 2, 8 + max(taps - 1, 1) * C, generator=g)
+    rows = torch.randperm(S + 2, generator=g)[:S].int()
+    qsl = torch.tensor([0] + lens).cumsum(0).int()
+    seq = torch.tensor([n + (0 if i % 2 else 9) for i, n in enumerate(lens)], dtype=torch.int32)
+    for single in ([0, 1] if max(lens) == 1 else [0]):
+        sc, sg = state.clone(), state.to(gpu)
+        want = seqmix.causal_conv(x, w, b, sc, rows, 8, qsl, seq, True, 1 if single else max(lens))
+        got = seqmix.causal_conv(x.to(gpu), w.to(gpu), b.to(gpu), sg, rows.to(gpu), 8, qsl.to(gpu), seq.to(gpu), True,
+                                 1 if single else max(lens))
+        torch.testing.assert_close(got.cpu().float(), want.float(), **tol(dt))
+        torch.testing.assert_close(sg.cpu(), sc, rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("N,groups,wn", [(16, 2, 16), (128, 16, 8), (384, 8, 48), (384, 3, 384), (2048, 16, 128), (4096, 8, 4096), (1024, 1, 1024),
+                                         (4096, 1, 4096), (8192, 2, 8192), (6144, 2, 6144)])
+def test_gated_norm_rows(gpu, dt, N, groups, wn):
+    g = torch.Generator().manual_seed(N + groups)
+    o, z, w = torch.randn(3, N, generator=g), torch.randn(3, N + 8, generator=g).to(dt)[:, 8:], torch.randn(wn, generator=g).to(dt)
+    for act, first in (("silu", True), ("sigmoid", False), ("silu", False)):
+        want, got = torch.zeros(3, N + 16, dtype=dt), torch.zeros(3, N + 16, dtype=dt, device=gpu)
+        seqmix.gated_norm(o, z, w, 1e-5, groups, act, first, dt, 0.5, want[:, 16:])
+        seqmix.gated_norm(o.to(gpu), z.to(gpu), w.to(gpu), 1e-5, groups, act, first, dt, 0.5, got[:, 16:])
+        torch.testing.assert_close(got.cpu().float(), want.float(), **tol(dt))
