@@ -26,8 +26,8 @@ void launch_gate_linear(float*, const void*, long, const void*, const void*, int
 void launch_kv_write(void*, long, const void*, long, const void*, long, const int64_t*, int, int, int, int, int, int,
                      int, bool, hipStream_t);
 bool launch_window_attention(void*, const void*, long, const void*, long, const int*, int, const int*, const int*, int,
-                             int, int, int, int, int, int, int, int, float, int, int, int, const float*, int, bool,
-                             hipStream_t);
+                             int, int, int, int, int, int, int, int, float, int, int, int, const float*, int, int, float*,
+                             bool, hipStream_t);
 bool launch_matrix_scan(float*, const void*, long, const void*, long, const void*, long, const float*, const float*,
                         float*, long, const int*, long, const int*, const int*, int, int, int, int, int, int, float,
                         float, bool, bool, int, int, float*, float*, long, hipStream_t);
@@ -179,13 +179,21 @@ void window_attention(at::Tensor out, at::Tensor q, at::Tensor cache, at::Tensor
               is_bf(out) == bf, "out: [T, H*dv]");
   TORCH_CHECK(block_tables.is_cuda() && block_tables.scalar_type() == at::kInt && block_tables.dim() == 2 &&
               block_tables.size(0) >= S && block_tables.stride(1) == 1, "block_tables: int32 [S, max_blocks]");
+  // a step of few rows splits its keys over workgroups
+  const int64_t span = block_tables.stride(0) * bs;
+  const int nsplit = !bf || dk > 128 || dv > 128 ? 1 :
+      mxs::row_attention_splits(T, static_cast<int>(H), static_cast<int>(G),
+                                window > 0 ? std::min(span, window + std::max<int64_t>(keep, 0)) : span);
+  at::Tensor part;
+  if (nsplit > 1) part = at::empty({T * H * nsplit * (dv + 2)}, out.options().dtype(at::kFloat));
   const bool ok = mxs::launch_window_attention(
       out.data_ptr(), mat(q, bf, T, H * dk, "q"), q.stride(0), cache.data_ptr(), cache.stride(0),
       block_tables.data_ptr<int>(), static_cast<int>(block_tables.stride(0)), i32(qsl, S + 1, "qsl"),
       i32(seq_lens, S, "seq_lens"), static_cast<int>(S), static_cast<int>(T), static_cast<int>(koff),
       static_cast<int>(voff), static_cast<int>(H), static_cast<int>(G), static_cast<int>(dk), static_cast<int>(dv),
       static_cast<int>(bs), static_cast<float>(scale), static_cast<int>(window), static_cast<int>(keep),
-      static_cast<int>(std::min<int64_t>(max_query_len, T)), sinkp, static_cast<int>(v_stride), bf, stream());
+      static_cast<int>(std::min<int64_t>(max_query_len, T)), sinkp, static_cast<int>(v_stride), nsplit,
+      nsplit > 1 ? part.data_ptr<float>() : nullptr, bf, stream());
   TORCH_CHECK(ok, "window_attention: head sizes beyond what the kernel holds (dv <= 512)");
 }
 

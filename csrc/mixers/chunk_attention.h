@@ -32,6 +32,13 @@ struct ChunkArgs {
 // false: head sizes that no kernel holds.  max_q: an upper bound of a sequence's rows in this launch.
 bool launch_chunk_attention(const ChunkArgs& a, int max_q, hipStream_t st);
 
+// Single rows (row_attention.hip): dk, dv multiples of 8 up to 128, q and the cache's pieces 16-byte aligned, bs (a power of
+// two) tokens a block, value rows vs apart.  nsplit stretches of the keys to a row, fp32 part [rows, H, nsplit, dv + 2] when
+// there are more than one.
+void launch_row_attention(const ChunkArgs& a, int rows, int bs, int vs, int nsplit, float* part, hipStream_t st);
+// how many stretches serve rows of at most `span` visible keys
+int row_attention_splits(long rows, int H, int G, long span);
+
 // base[s]: row of key position 0 of sequence s when the keys its chunk sees (with window > 0: from the page of the first
 // query's oldest one) lie back to back, offs[s]: its first row; offs[S]: rows in all.
 void launch_latent_plan(int* base, int* offs, const int* qsl, const int* seq_lens, int S, int window, hipStream_t st);

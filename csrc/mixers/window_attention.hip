@@ -251,31 +251,38 @@ __global__ void __launch_bounds__(256) window_attention_rows_kernel(
 bool launch_window_attention(void* out, const void* q, long q_stride, const void* cache, long block_stride,
                              const int* block_tables, int bt_stride, const int* qsl, const int* seq_lens, int S,
                              int rows, int koff, int voff, int H, int G, int dk, int dv, int bs, float scale,
-                             int window, int keep, int max_q, const float* sink, int vs, bool bf, hipStream_t st) {
+                             int window, int keep, int max_q, const float* sink, int vs, int nsplit, float* part,
+                             bool bf, hipStream_t st) {
   if (rows == 0 || S == 0) return true;
   if (vs <= 0) vs = dv;  // value rows back to back
-  // prompt chunks in bf16 with MFMA-shaped heads: the matrix-core form (rows of a mixed step's single
-  // tokens ride along as tiles of one row); everything else the forms above
-  if (bf && vs == dv && max_q >= 16 && bs == 16 && dk % 16 == 0 && dv % 16 == 0 && dk <= 128 && dv <= 128 && q_stride % 4 == 0 &&
-      reinterpret_cast<uintptr_t>(q) % 8 == 0 && koff % 8 == 0 && voff % 8 == 0 && block_stride % 8 == 0) {
-    ChunkArgs a{};
-    a.out = (bf16_t*)out;
-    a.q = (const bf16_t*)q;
-    a.q_stride = q_stride;
-    a.qsl = qsl;
-    a.seq_lens = seq_lens;
-    a.S = S; a.H = H; a.G = G; a.dk = dk; a.dv = dv;
-    a.scale = scale;
-    a.window = window;
-    a.keep = keep;
-    a.sink = sink;
-    a.cache = (const bf16_t*)cache;
-    a.block_stride = block_stride;
-    a.block_tables = block_tables;
-    a.bt_stride = bt_stride;
-    a.koff = koff;
-    a.voff = voff;
+  // bf16 with heads of whole 16-byte pieces: the matrix-core forms, for prompt chunks (rows of a mixed step's single tokens
+  // ride along as tiles of one row) and for steps of short chunks and single tokens; everything else the forms above
+  ChunkArgs a{};
+  a.out = (bf16_t*)out;
+  a.q = (const bf16_t*)q;
+  a.q_stride = q_stride;
+  a.qsl = qsl;
+  a.seq_lens = seq_lens;
+  a.S = S; a.H = H; a.G = G; a.dk = dk; a.dv = dv;
+  a.scale = scale;
+  a.window = window;
+  a.keep = keep;
+  a.sink = sink;
+  a.cache = (const bf16_t*)cache;
+  a.block_stride = block_stride;
+  a.block_tables = block_tables;
+  a.bt_stride = bt_stride;
+  a.koff = koff;
+  a.voff = voff;
+  const bool pieces = bf && dk <= 128 && dv <= 128 && koff % 8 == 0 && voff % 8 == 0 && block_stride % 8 == 0;
+  if (pieces && vs == dv && max_q >= 16 && bs == 16 && dk % 16 == 0 && dv % 16 == 0 && q_stride % 4 == 0 &&
+      reinterpret_cast<uintptr_t>(q) % 8 == 0)
     return launch_chunk_attention(a, max_q, st);
+  if (pieces && dk % 8 == 0 && dv % 8 == 0 && vs % 8 == 0 && (bs & (bs - 1)) == 0 && q_stride % 8 == 0 &&
+      reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(cache) % 16 == 0) {
+    launch_row_attention(a, rows, bs, vs, part ? nsplit : 1, part, st);
+    MXS_CHECK_LAUNCH();
+    return true;
   }
   if (dv > 64 * kMaxVChunks) return false;
   const int el = bf ? 8 : 4;  // elements per 16-byte load
