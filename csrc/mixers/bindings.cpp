@@ -1,5 +1,7 @@
 // torch bindings of the mixer kernels (mxserve/_M): shape and dtype checks on the host, so that a
 // launch never reads or writes outside what the kernels and their grids assume.
+#include <limits>
+
 #include "chunk_attention.h"
 #include "bind_util.h"
 #include "column_scan.h"
@@ -61,7 +63,8 @@ void launch_rope_half_into(void*, long, const void*, long, const int64_t*, int, 
 void launch_route_topk(float*, int*, const float*, int, int, int, bool, bool, hipStream_t);
 void launch_capped_glu(void*, const void*, long, int, int, float, float, bool, hipStream_t);
 bool launch_expert_align(int*, int*, const int*, int, int, hipStream_t);
-void launch_gather_scaled(void*, const void*, long, const float*, const int*, int, int, int, bool, hipStream_t);
+void launch_gather_scaled(void*, const void*, long, const float*, const int*, int, int, int, const int*, const int*, int, int,
+                          int*, bool, hipStream_t);
 void launch_spread_scaled(void*, const void*, long, const float*, const int*, int, int, int, int, bool, hipStream_t);
 void launch_expert_combine(void*, const void*, const int*, int, int, long, const void*, long, int, const float*, bool, bool,
                            hipStream_t);
@@ -726,7 +729,25 @@ void gather_scaled(at::Tensor xs, at::Tensor h, OptT w, at::Tensor inv, int64_t 
               is_bf(xs) == bf, "xs: contiguous [T*k, W]");
   // inv comes from expert_align over the same pairs: a permutation of 0 .. T*k-1
   mxs::launch_gather_scaled(xs.data_ptr(), mat(h, bf, T, W, "h"), h.stride(0), wp, i32(inv, T * k, "inv"),
-                            static_cast<int>(T * k), static_cast<int>(k), static_cast<int>(W), bf, stream());
+                            static_cast<int>(T * k), static_cast<int>(k), static_cast<int>(W), nullptr, nullptr, 0, 0, nullptr, bf,
+                            stream());
+}
+
+void gather_slabs(at::Tensor xs, at::Tensor index, at::Tensor h, OptT w, at::Tensor ids, at::Tensor offs, at::Tensor inv) {
+  const bool bf = is_bf(h);
+  TORCH_CHECK(h.dim() == 2 && ids.dim() == 2 && ids.size(0) == h.size(0) && xs.dim() == 3, "h [T, W], ids [T, k], xs [E, cap, W]");
+  const int64_t T = h.size(0), W = h.size(1), k = ids.size(1), E = xs.size(0), cap = xs.size(1);
+  const float* wp = nullptr;
+  if (w.has_value()) {
+    TORCH_CHECK(w->dim() == 2 && w->size(0) == T && w->size(1) == k, "w [T, k]");
+    wp = f32(*w, "w");
+  }
+  TORCH_CHECK(xs.is_cuda() && xs.is_contiguous() && xs.size(2) == W && is_bf(xs) == bf, "xs: contiguous [E, cap, W]");
+  TORCH_CHECK(E * cap <= std::numeric_limits<int>::max(), "more rows than an int32 index holds");
+  TORCH_CHECK(index.is_cuda() && index.is_contiguous() && index.scalar_type() == at::kInt && index.numel() == T * k, "index int32 [T*k]");
+  mxs::launch_gather_scaled(xs.data_ptr(), mat(h, bf, T, W, "h"), h.stride(0), wp, i32(inv, T * k, "inv"),
+                            static_cast<int>(T * k), static_cast<int>(k), static_cast<int>(W), i32(ids, T * k, "ids"),
+                            i32(offs, E + 1, "offs"), static_cast<int>(E), static_cast<int>(cap), index.data_ptr<int>(), bf, stream());
 }
 
 void spread_scaled(at::Tensor xs, at::Tensor h, OptT w, at::Tensor ids) {
@@ -915,6 +936,7 @@ PYBIND11_MODULE(_M, m) {
   m.def("capped_glu", &capped_glu);
   m.def("expert_align", &expert_align);
   m.def("gather_scaled", &gather_scaled);
+  m.def("gather_slabs", &gather_slabs);
   m.def("spread_scaled", &spread_scaled);
   m.def("expert_combine", &expert_combine);
   m.def("embed_normed", &embed_normed);

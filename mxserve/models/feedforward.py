@@ -111,12 +111,19 @@ class RoutedExperts(FeedForward):
                 and no host round trip, so a captured single-token step can replay it; E / top times
                 the needed products, which steps of a few tokens do not feel (they stream the
                 experts' weights either way)
-      sorted    rows sorted by expert (expert_align, gather_scaled), one product pair per expert that
-                got rows (one host read of the E + 1 offsets), expert_combine gathers each token's rows
+      sorted    rows sorted by expert (expert_align; one host read of the E + 1 offsets) into slabs as long as the
+                fullest expert, again two batched products; or, where the slabs would be mostly empty, one product pair per
+                expert that got rows.  expert_combine gathers each token's rows
     """
 
     BATCHED_MAX_TOKENS = 32    # always batched up to this many tokens ...
     BATCHED_MAX_ROWS = 1024    # ... and beyond while experts x tokens stays within this many rows
+    # Sorted rows: an expert's own two products take no less than about 40 us, however few its rows (and half as long again as
+    # its share of a batched product when it has a thousand: they fill a third of the chip).  8 experts of 2,048 x 2,560,
+    # even choices, products alone: 64 tokens 333 us one by one, 49 us in slabs; 512 tokens 332 / 80; 2,048: 353 / 141;
+    # 4,096: 435 / 273.  So slabs, until their empty rows (at a large product's rate) and the weights of experts without rows
+    # (at the memory's) cost more than 30 us for each expert that has some.
+    SLAB_GAIN_S, SLAB_FLOPS, SLAB_BYTES = 30e-6, 1e15, 5e12
 
     def __init__(self, prefix: str, width: int, experts: int, top: int, ff: int, limit: Optional[float],
                  shared: Optional[FeedForward] = None, alpha: float = 1.702, renorm: bool = False,
@@ -218,9 +225,18 @@ class RoutedExperts(FeedForward):
             return seqmix.ExpertRows(ys, ids.reshape(-1), self.top, T, extra, row_stride=T, weights=w_out, by_expert=True,
                                      gate=gate)
         offs, inv = seqmix.expert_align(ids, self.E)
+        o = offs.tolist()  # the one host read of this path
+        counts = [b - a for a, b in zip(o, o[1:])]
+        cap, used = max(counts), sum(n > 0 for n in counts)
+        per_row = up[0].numel() + down[0].numel()  # multiply-adds of a row, weights of an expert
+        if (2.0 * per_row * (self.E * cap - o[-1]) / self.SLAB_FLOPS
+                + per_row * up.element_size() * (self.E - used) / self.SLAB_BYTES) <= self.SLAB_GAIN_S * used:
+            xs, index = seqmix.gather_slabs(h, w_in, ids, offs, inv, cap)
+            a = self.act(torch.bmm(xs, up).view(self.E * cap, -1))
+            ys = torch.bmm(a.view(self.E, cap, -1), down)
+            return seqmix.ExpertRows(ys, index, self.top, T, extra, weights=w_out, gate=gate)
         xs = seqmix.gather_scaled(h, w_in, inv, self.top)
         ys = torch.empty_like(xs)
-        o = offs.tolist()  # the one host read of this path
         for e in range(self.E):
             a0, a1 = o[e], o[e + 1]
             if a1 > a0:

@@ -1369,6 +1369,25 @@ def gather_scaled(h: torch.Tensor, weights: Optional[torch.Tensor], inv: torch.T
     return xs
 
 
+def gather_slabs(h: torch.Tensor, weights: Optional[torch.Tensor], ids: torch.Tensor, offs: torch.Tensor, inv: torch.Tensor,
+                 cap: int) -> tuple:
+    """(xs [E, cap, W], index int32 [T*k]): gather_scaled's rows with expert e's from row e * cap on, for a batched product
+    over all experts; index[p] is pair p's row of the [E * cap, W] stack.  offs, inv from expert_align over ids; cap is at
+    least every expert's count.  Rows behind an expert's last one are not written."""
+    (T, k), E = ids.shape, offs.numel() - 1
+    if _gpu(h):
+        xs = torch.empty(E, int(cap), h.shape[1], dtype=h.dtype, device=h.device)
+        index = torch.empty(T * k, dtype=torch.int32, device=h.device)
+        ext().gather_slabs(xs, index, h, weights, ids, offs, inv)
+        return xs, index
+    rows = gather_scaled(h, weights, inv, k)
+    flat = ids.reshape(-1).long()
+    index = flat * int(cap) + inv.long() - offs.long()[flat]
+    xs = torch.zeros(E * int(cap), h.shape[1], dtype=h.dtype)
+    xs[index] = rows[inv.long()]
+    return xs.view(E, int(cap), -1), index.to(torch.int32)
+
+
 def spread_scaled(h: torch.Tensor, weights: Optional[torch.Tensor], ids: torch.Tensor, num_experts: int) -> torch.Tensor:
     """[E, T, W]: row (e, t) = weights[t, j] * h[t] where ids[t, j] = e, zeros for the experts a token
     did not choose (the experts' inputs for a batched product over all experts, no sorting).
