@@ -1,5 +1,6 @@
 // Arguments of the column scans (csrc/mixers/column_scan.hip), shared with the torch bindings.
 #pragma once
+#include <hip/hip_runtime.h>
 
 namespace mxs {
 
@@ -38,5 +39,9 @@ struct ScanArgs {
   float* sc_start;   // [S, npieces, H*dv*dk]
   float* sc_decay;   // state space: [S, npieces, H], summed decay exponents; gated linear: [S, npieces, H*dk], summed logs
 };
+
+// the state space in chunks on the matrix cores (ssd_chunk.hip): one pass, mode and pieces as above
+bool ssd_chunk_fits(const ScanArgs& a, int S);
+bool launch_ssd_chunk(const ScanArgs& a, int S, hipStream_t st);
 
 }  // namespace mxs

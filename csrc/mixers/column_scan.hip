@@ -472,6 +472,7 @@ static bool launch_cs(const ScanArgs& a, int S, hipStream_t st) {
 static bool launch_pass(const ScanArgs& a, int S, int kind, bool bf, hipStream_t st) {
   if (kind == kDeltaRule) return bf ? launch_cs<bf16_t, kDeltaRule>(a, S, st) : launch_cs<float, kDeltaRule>(a, S, st);
   if (kind == kGatedLinear) return bf ? launch_cs<bf16_t, kGatedLinear>(a, S, st) : launch_cs<float, kGatedLinear>(a, S, st);
+  if (bf && ssd_chunk_fits(a, S)) return launch_ssd_chunk(a, S, st);
   return bf ? launch_cs<bf16_t, kStateSpace>(a, S, st) : launch_cs<float, kStateSpace>(a, S, st);
 }
 

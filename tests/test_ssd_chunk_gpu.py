@@ -1,0 +1,66 @@
+"""The state space in chunks on the matrix cores against the recurrence in 64 bits: chunk counts around tiles and pieces, heads
+of every size that fills a workgroup, states that go on from a slot, and decays from almost none to a full reset per token."""
+import pytest
+import torch
+
+from mxserve.ops import seqmix
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(x, B, C, dt, dtb, A, D, state, before, new, G):
+    """[T, H, P], [T, G, N] .. in 64 bits, state [S, H, P, N] in place -> y [T, H, P]."""
+    H = x.shape[1]
+    y, t = torch.empty_like(x), 0
+    d = torch.nn.functional.softplus(dt + dtb, threshold=1e9)
+    a = torch.exp(-torch.exp(A) * d)
+    B, C = B.repeat_interleave(H // G, 1), C.repeat_interleave(H // G, 1)
+    for s, n in enumerate(new):
+        if before[s] == 0:
+            state[s] = 0
+        for _ in range(n):
+            state[s] = a[t].view(H, 1, 1) * state[s] + (d[t].view(H, 1) * x[t]).unsqueeze(2) * B[t].unsqueeze(1)
+            y[t] = (state[s] * C[t].unsqueeze(1)).sum(-1) + D.view(H, 1) * x[t]
+            t += 1
+    return y
+
+
+def run(gpu, H, G, N, P, before, new, a_mean, seed=0):
+    g = torch.Generator().manual_seed(seed + N + P)
+    T, S, off = sum(new), len(new), 4
+    x, B, C, dt = (torch.randn(T, n + 8, generator=g).mul(m).bfloat16()[:, 8:] for n, m in ((H * P, 1), (G * N, 0.3), (G * N, 0.3), (H, 1)))
+    dtb, A, D = torch.randn(H, generator=g) - 1.0, torch.randn(H, generator=g) * 0.5 + a_mean, torch.randn(H, generator=g)
+    pool = torch.randn(S + 1, off + H * P * N + 4, generator=g)
+    rows = torch.randperm(S + 1, generator=g)[:S].int()
+    qsl = torch.tensor([0] + new).cumsum(0).int()
+    lens = torch.tensor([b + n for b, n in zip(before, new)], dtype=torch.int32)
+    dev = [t.to(gpu) for t in (dtb, A, D)]
+    gp = pool.to(gpu)
+    on = lambda t: torch.cat([torch.zeros(T, 8, dtype=t.dtype), t], 1).to(gpu)[:, 8:]  # noqa: E731  (keeps the row stride)
+    y = seqmix.ssd_scan(on(x), on(B), on(C), on(dt), *dev, gp, rows.to(gpu), off, qsl.to(gpu), lens.to(gpu), H, G, N, P, max(new))
+    st = pool[rows.long(), off:off + H * P * N].double().view(S, H, P, N)
+    want = reference(x.double().view(T, H, P), B.double().view(T, G, N), C.double().view(T, G, N), dt.double(), dtb.double(), A.double(),
+                     D.double(), st, before, new, G)
+    got_st = gp.cpu()[rows.long(), off:off + H * P * N].double().view(S, H, P, N)
+    return y.cpu().double().view(T, H, P), want, got_st, st, gp.cpu(), pool, rows
+
+
+@pytest.mark.parametrize("H,G,N,P", [(2, 1, 128, 64), (8, 2, 64, 32), (2, 2, 128, 128), (4, 2, 64, 64), (8, 1, 128, 32)])
+@pytest.mark.parametrize("before,new", [([5], [63]), ([0], [64]), ([0, 9, 0], [64, 65, 1]), ([3], [127]), ([0, 7], [300, 128]),
+                                        ([1, 0, 2, 0], [1, 140, 1, 257]), ([0, 4, 4, 4], [16, 15, 17, 33])])
+def test_chunks(gpu, H, G, N, P, before, new):
+    y, want, st, wst, pool, old, rows = run(gpu, H, G, N, P, before, new, -1.5)
+    # fp32 sums over up to 300 tokens and 128 channels: a few hundred roundings of 2^-24, walking at random, on terms of size 30
+    torch.testing.assert_close(y, want, rtol=1e-5, atol=1e-4)
+    torch.testing.assert_close(st, wst, rtol=1e-5, atol=1e-4)
+    spare = [r for r in range(old.shape[0]) if r not in rows.tolist()]
+    assert torch.equal(pool[spare], old[spare])  # other slots and the slots' borders stay
+    assert torch.equal(pool[:, :4], old[:, :4]) and torch.equal(pool[:, -4:], old[:, -4:])
+
+
+@pytest.mark.parametrize("a_mean", [-12.0, 3.0, 7.0])
+def test_decays(gpu, a_mean):
+    """Half lives of a thousand tokens, and resets within a few or one, where the running sum of exponents is in the thousands."""
+    y, want, st, wst, *_ = run(gpu, 4, 2, 128, 64, [9, 0], [200, 150], a_mean)
+    torch.testing.assert_close(y, want, rtol=1e-5, atol=2e-4)
+    torch.testing.assert_close(st, wst, rtol=1e-5, atol=2e-4)
