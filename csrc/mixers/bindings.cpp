@@ -326,7 +326,7 @@ void column_scan(int kind, at::Tensor out, at::Tensor q, at::Tensor k, at::Tenso
                  OptT dt_bias, OptT A_log, OptT D, at::Tensor state, at::Tensor state_rows, int64_t off,
                  at::Tensor qsl, at::Tensor seq_lens, int64_t H, int64_t G, int64_t dk, int64_t dv, double q_scale,
                  double unit_eps, int64_t piece = 1, int64_t npieces = 1, OptT sc_local = OptT(), OptT sc_start = OptT(),
-                 OptT sc_decay = OptT(), int64_t mode = 0, int64_t max_q = 0) {
+                 OptT sc_decay = OptT(), int64_t mode = 0, int64_t max_q = 0, OptT work = OptT()) {
   const bool bf = is_bf(q), delta = kind == mxs::kDeltaRule, gla = kind == mxs::kGatedLinear;
   const int64_t T = q.size(0), S = seq_lens.numel();
   TORCH_CHECK(G >= 1 && H % G == 0, "heads must divide over the q/k heads (groups)");
@@ -390,6 +390,11 @@ void column_scan(int kind, at::Tensor out, at::Tensor q, at::Tensor k, at::Tenso
     p.sc_start = f32(*sc_start, "sc_start");
     p.sc_decay = delta ? nullptr : f32(*sc_decay, "sc_decay");
   }
+  if (work.has_value()) {
+    const int64_t floats = mxs::delta_chunk_floats(p.dk, p.dv);
+    TORCH_CHECK(delta && bf && floats > 0 && work->numel() >= (T / 32 + S) * H * floats, "delta rule in chunks: bf16, its sizes, its scratch");
+    if (S == 0 || T == 0 || mxs::launch_delta_chunk(p, static_cast<int>(S), f32(*work, "work"), stream())) return;
+  }
   TORCH_CHECK(mxs::launch_column_scan(p, static_cast<int>(S), kind, bf, stream()), "column scan: key / state size beyond 256");
 }
 
@@ -404,9 +409,9 @@ void ssd_scan(at::Tensor out, at::Tensor x, at::Tensor B, at::Tensor C, at::Tens
 void delta_scan(at::Tensor out, at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor beta, at::Tensor a, at::Tensor dt_bias,
                 at::Tensor A_log, at::Tensor state, at::Tensor state_rows, int64_t off, at::Tensor qsl, at::Tensor seq_lens,
                 int64_t H, int64_t G, int64_t dk, int64_t dv, double q_scale, double unit_eps, int64_t mode, int64_t piece,
-                int64_t npieces, OptT sc_local, OptT sc_start, int64_t max_q) {
+                int64_t npieces, OptT sc_local, OptT sc_start, int64_t max_q, OptT work) {
   column_scan(mxs::kDeltaRule, out, q, k, v, OptT(beta), OptT(a), OptT(dt_bias), OptT(A_log), OptT(), state, state_rows, off, qsl, seq_lens, H, G, dk, dv,
-              q_scale, unit_eps, piece, npieces, sc_local, sc_start, OptT(), mode, max_q);
+              q_scale, unit_eps, piece, npieces, sc_local, sc_start, OptT(), mode, max_q, work);
 }
 
 void gla_scan(at::Tensor out, at::Tensor q, at::Tensor k, at::Tensor v, at::Tensor loga, at::Tensor state,
@@ -929,6 +934,7 @@ PYBIND11_MODULE(_M, m) {
   m.def("gated_norm", &gated_norm);
   m.def("ssd_scan", &ssd_scan);
   m.def("delta_scan", &delta_scan);
+  m.def("delta_chunk_floats", [](int64_t dk, int64_t dv) { return mxs::delta_chunk_floats(static_cast<int>(dk), static_cast<int>(dv)); });
   m.def("latent_prep", &latent_prep);
   m.def("rope_half_into", &rope_half_into);
   m.def("latent_attention", &latent_attention);

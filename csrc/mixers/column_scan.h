@@ -44,4 +44,9 @@ struct ScanArgs {
 bool ssd_chunk_fits(const ScanArgs& a, int S);
 bool launch_ssd_chunk(const ScanArgs& a, int S, hipStream_t st);
 
+// the delta rule in chunks (delta_chunk.hip): floats of scratch for each of rows / 32 + S chunks and head (0: sizes that it does
+// not hold), and the whole scan; false: operands that it does not take
+long delta_chunk_floats(int dk, int dv);
+bool launch_delta_chunk(const ScanArgs& a, int S, float* work, hipStream_t st);
+
 }  // namespace mxs

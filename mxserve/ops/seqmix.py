@@ -1007,6 +1007,11 @@ def ssd_scan(x: torch.Tensor, B: torch.Tensor, C: torch.Tensor, dt: torch.Tensor
     return out.reshape(T, H * P)
 
 
+# A bf16 step of the delta rule runs in chunks when its longest chunk holds this many tokens, and more for each sequence: token
+# by token a step takes 0.45 us for each token of its longest chunk, in chunks 30 us and 2.7 us a sequence before anything else.
+# 16 heads of 128, token by token / in chunks: one chunk of 64 34 / 42 us, 127 62 / 47, 512 260 / 79, 4,096 1,480 / 437; 32
+# chunks of 16 65 / 97; a chunk beside 32 single tokens: of 200 112 / 115, of 400 203 / 124.
+DELTA_CHUNK_TOKENS, DELTA_CHUNK_TOKENS_PER_SEQ = 64, 6
 DELTA_MIN_PIECES = 4  # a split delta-rule scan does three times the work: fewer pieces do not pay
 
 
@@ -1026,7 +1031,8 @@ def delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Te
     pieces that run side by side, pass 1 giving every piece's L (end state from an empty start) and P
     (dk more state columns started as the identity and fed no values), the states at the pieces'
     starts following by one fp32 matrix product per piece, pass 2 writing the outputs.  Three times
-    the multiply-adds, but DELTA_MIN_PIECES or more pieces at once instead of one serial walk."""
+    the multiply-adds, but DELTA_MIN_PIECES or more pieces at once instead of one serial walk.
+    bf16 steps with a long chunk run in chunks of 32 tokens on the matrix cores instead (csrc/mixers/delta_chunk.hip)."""
     T = q.shape[0]
     H, G = num_heads, qk_heads
     if _gpu(q):
@@ -1034,21 +1040,27 @@ def delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Te
         S = seq_lens.numel()
         args = (out, q, k, v, beta, a, dt_bias, A_log, state, state_rows, int(off), qsl, seq_lens, H, G, dk, dv,
                 float(q_scale), float(unit_eps))
+        if q.dtype == torch.bfloat16 and min(max_query_len, T) >= DELTA_CHUNK_TOKENS + DELTA_CHUNK_TOKENS_PER_SEQ * S:
+            floats = ext().delta_chunk_floats(dk, dv) * (T // 32 + S) * H
+            if 0 < 4 * floats <= SCAN_SCRATCH_BYTES and state.data_ptr() % 16 == 0 and state.stride(0) % 4 == 0 and off % 4 == 0:
+                work = torch.empty(floats, dtype=torch.float32, device=q.device)
+                ext().delta_scan(*args, 0, 1, 1, None, None, int(max_query_len), work)
+                return out
         piece, npieces, _, _ = _scan_split(S, T, max_query_len, H * (dv + dk) * dk, H, 4 * (dv + dk), q.device)
         if npieces < DELTA_MIN_PIECES:
-            ext().delta_scan(*args, 0, 1, 1, None, None, int(max_query_len))
+            ext().delta_scan(*args, 0, 1, 1, None, None, int(max_query_len), None)
             return out
         n = H * dv * dk
         loc = torch.empty(S, npieces, H, dv + dk, dk, dtype=torch.float32, device=q.device)
         start = torch.empty(S, npieces, H * dv, dk, dtype=torch.float32, device=q.device)
-        ext().delta_scan(*args, 1, piece, npieces, loc, start, int(max_query_len))
+        ext().delta_scan(*args, 1, piece, npieces, loc, start, int(max_query_len), None)
         first = (seq_lens - (qsl[1:] - qsl[:-1]) <= 0).view(S, 1, 1)
         slot = state.index_select(0, state_rows.long())[:, off:off + n].view(S, H * dv, dk)
         start[:, 0] = torch.where(first, torch.zeros((), dtype=torch.float32, device=q.device), slot)
         for p in range(npieces - 1):  # St' = St Pt + Lt in the transposed storage, batched over sequences and heads
             start[:, p + 1] = torch.baddbmm(loc[:, p, :, :dv].reshape(S * H, dv, dk), start[:, p].reshape(S * H, dv, dk),
                                             loc[:, p, :, dv:].reshape(S * H, dk, dk)).view(S, H * dv, dk)
-        ext().delta_scan(*args, 2, piece, npieces, loc, start, int(max_query_len))
+        ext().delta_scan(*args, 2, piece, npieces, loc, start, int(max_query_len), None)
         return out
     out = torch.zeros(T, H, dv, dtype=torch.float32)
     rep = H // G
