@@ -49,4 +49,7 @@ bool launch_ssd_chunk(const ScanArgs& a, int S, hipStream_t st);
 long delta_chunk_floats(int dk, int dv);
 bool launch_delta_chunk(const ScanArgs& a, int S, float* work, hipStream_t st);
 
+// steps of single tokens (step_scan.hip); false: sizes or a state that it does not take
+bool launch_step_scan(const ScanArgs& a, int S, int kind, bool bf, hipStream_t st);
+
 }  // namespace mxs

@@ -483,6 +483,7 @@ bool launch_column_scan(const ScanArgs& a0, int S, int kind, bool bf, hipStream_
     a.mode = 0;
     a.piece = 1;
     a.npieces = 1;
+    if (a.max_q == 1 && launch_step_scan(a, S, kind, bf, st)) return true;
     return launch_pass(a, S, kind, bf, st);
   }
   // the delta rule's step is no diagonal map of the state: the caller runs its passes one by one and
