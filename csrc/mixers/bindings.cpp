@@ -162,7 +162,7 @@ void kv_write(at::Tensor cache, at::Tensor k, at::Tensor v, at::Tensor slots, in
 void window_attention(at::Tensor out, at::Tensor q, at::Tensor cache, at::Tensor block_tables, at::Tensor qsl,
                       at::Tensor seq_lens, int64_t koff, int64_t voff, int64_t H, int64_t G, int64_t dk, int64_t dv,
                       int64_t bs, double scale, int64_t window, int64_t keep, int64_t max_query_len, OptT sink,
-                      int64_t v_stride) {
+                      int64_t v_stride, int64_t max_seq_len) {
   const bool bf = is_bf(q);
   const float* sinkp = nullptr;
   if (sink.has_value()) {
@@ -182,13 +182,14 @@ void window_attention(at::Tensor out, at::Tensor q, at::Tensor cache, at::Tensor
               is_bf(out) == bf, "out: [T, H*dv]");
   TORCH_CHECK(block_tables.is_cuda() && block_tables.scalar_type() == at::kInt && block_tables.dim() == 2 &&
               block_tables.size(0) >= S && block_tables.stride(1) == 1, "block_tables: int32 [S, max_blocks]");
-  // a step of few rows splits its keys over workgroups
-  const int64_t span = block_tables.stride(0) * bs;
+  // a step of few rows, and the long walks of few chunks, split their keys over workgroups
+  const int64_t table = block_tables.stride(0) * bs, seen = window > 0 ? window + std::max<int64_t>(keep, 0) : table;
+  const int h = static_cast<int>(H), g = static_cast<int>(G);
   const int nsplit = !bf || dk > 128 || dv > 128 ? 1 :
-      mxs::row_attention_splits(T, static_cast<int>(H), static_cast<int>(G),
-                                window > 0 ? std::min(span, window + std::max<int64_t>(keep, 0)) : span);
+      std::min(max_query_len, T) < 16 ? mxs::row_attention_splits(T, h, g, std::min(table, seen)) :
+      mxs::chunk_attention_splits(T, static_cast<int>(S), h, g, static_cast<int>(dk), static_cast<int>(dv), std::min(max_seq_len, seen));
   at::Tensor part;
-  if (nsplit > 1) part = at::empty({T * H * nsplit * (dv + 2)}, out.options().dtype(at::kFloat));
+  if (nsplit > 1) part = at::empty({T * H * nsplit * (dv + 4)}, out.options().dtype(at::kFloat));
   const bool ok = mxs::launch_window_attention(
       out.data_ptr(), mat(q, bf, T, H * dk, "q"), q.stride(0), cache.data_ptr(), cache.stride(0),
       block_tables.data_ptr<int>(), static_cast<int>(block_tables.stride(0)), i32(qsl, S + 1, "qsl"),
@@ -644,7 +645,7 @@ void latent_rows(at::Tensor out, at::Tensor cache, at::Tensor block_tables, at::
 
 bool expanded_attention(at::Tensor out, at::Tensor q, at::Tensor kv, at::Tensor rows, at::Tensor base, at::Tensor qsl,
                         at::Tensor seq_lens, int64_t H, int64_t dn, int64_t dr, int64_t dv, int64_t rank, double scale,
-                        int64_t max_query_len, OptT sink, int64_t window) {
+                        int64_t max_query_len, OptT sink, int64_t window, int64_t max_seq_len) {
   const int64_t T = q.size(0), S = seq_lens.numel(), n = kv.size(0);
   TORCH_CHECK(window >= 0 && window < (1LL << 30) && H >= 1 && dn >= 8 && dr >= 8 && dv >= 16, "head sizes out of range");
   mxs::ChunkArgs a{};
@@ -675,6 +676,13 @@ bool expanded_attention(at::Tensor out, at::Tensor q, at::Tensor kv, at::Tensor 
   a.scale = static_cast<float>(scale);
   a.window = static_cast<int>(window);
   a.sink = f32n(sink, H, "sink");
+  a.rows = static_cast<int>(T);
+  a.nsplit = mxs::chunk_attention_splits(T, a.S, a.H, a.G, a.dk, a.dv, window > 0 ? std::min(max_seq_len, window) : max_seq_len);
+  at::Tensor part;
+  if (a.nsplit > 1) {
+    part = at::empty({T * H * a.nsplit * (dv + 4)}, out.options().dtype(at::kFloat));
+    a.part = part.data_ptr<float>();
+  }
   return mxs::launch_chunk_attention(a, static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(max_query_len, T))), stream());
 }
 

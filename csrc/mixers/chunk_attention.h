@@ -27,10 +27,17 @@ struct ChunkArgs {
   long x_stride, r_stride;
   const int* base;
   int dn, nrows;
+  // the walks of long tiles in nsplit stretches (rows: of the whole launch), fp32 part [rows, H, nsplit, dv + 4]; 0, 1: none
+  int rows, nsplit;
+  float* part;
 };
 
 // false: head sizes that no kernel holds.  max_q: an upper bound of a sequence's rows in this launch.
 bool launch_chunk_attention(const ChunkArgs& a, int max_q, hipStream_t st);
+// how many stretches serve a launch whose queries see `span` keys at most (0: not known)
+int chunk_attention_splits(long rows, int S, int H, int G, int dk, int dv, long span);
+// merges the records (maximum in log2 units, sum, two unused, output[width]) of rows: (token, head) pairs (latent_attention.hip)
+bool launch_attention_combine(void* out, const float* part, long rows, int nsplit, int width, hipStream_t st);
 
 // Single rows (row_attention.hip): dk, dv multiples of 8 up to 128, q and the cache's pieces 16-byte aligned, bs (a power of
 // two) tokens a block, value rows vs apart.  nsplit stretches of the keys to a row, fp32 part [rows, H, nsplit, dv + 2] when

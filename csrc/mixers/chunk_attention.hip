@@ -46,16 +46,18 @@ __device__ __forceinline__ float across(float v, bool sum) {  // with the lane 3
   return sum ? a + b : fmaxf(a, b);
 }
 
+constexpr int kSplitKeys = 768;  // shorter walks are one stretch's alone
+
 // DKP, DVP: head sizes the registers are laid out for (smaller ones ride in zeroed columns); KT: keys of a tile; PAGED:
 // where keys and values are.
-template <int DKP, int DVP, int KT, bool PAGED>
+template <int DKP, int DVP, int KT, bool PAGED, bool SPLIT>
 __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention_kernel(ChunkArgs a) {
   constexpr int KS = DKP / 16, DT = DVP / 32, KU = KT / 32;
   constexpr int KROW = DKP + 8, VROW = DVP + 8;  // padded by 16 bytes: neighbouring rows start in other banks
   constexpr int NK = KT * DKP / 8 / 256, NV = KT * DVP / 8 / 256;  // 16-byte pieces a thread stages
   static_assert(NK * 256 * 8 == KT * DKP && NV * 256 * 8 == KT * DVP, "tile");
   __shared__ __attribute__((aligned(16))) bf16_t lds[2][KT * (KROW + VROW)];
-  const int g = blockIdx.x, s = blockIdx.z;
+  const int g = blockIdx.x, s = SPLIT ? blockIdx.z / a.nsplit : blockIdx.z, stretch = SPLIT ? blockIdx.z - s * a.nsplit : 0;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int c = lane & 31, hi = lane >> 5;
   const int row0 = a.qsl[s], qlen = a.qsl[s + 1] - row0;
@@ -107,6 +109,23 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
   const int ntile = nA + glast / KT - t0 + 1;
   auto start_of = [&](int it) { return (it < nA ? it : t0 + it - nA) * KT; };
 
+  // this workgroup's tiles: all, or its stretch of a long walk (short walks are the first stretch's alone)
+  int it0 = 0, itn = ntile;
+  float* pp = nullptr;
+  if constexpr (SPLIT) {
+    pp = a.part + ((static_cast<long>(row0 + qi) * a.H + head) * a.nsplit + stretch) * (dv + 4);
+    if (ntile * KT >= kSplitKeys) {
+      it0 = ntile * stretch / a.nsplit;
+      itn = ntile * (stretch + 1) / a.nsplit;
+    } else if (stretch > 0) {
+      if (qok && hi == 0) {
+        pp[0] = -INFINITY;
+        pp[1] = 0.f;
+      }
+      return;
+    }
+  }
+
   const int* bt = PAGED ? a.block_tables + static_cast<long>(s) * a.bt_stride : nullptr;
   const int lastpage = PAGED ? min(glast >> 4, a.bt_stride - 1) : 0;
   const int dense0 = PAGED ? 0 : a.base[s];
@@ -154,9 +173,9 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
     for (int i = 0; i < NV; ++i)
       if (vrow[i] >= 0) *reinterpret_cast<uint4*>(buf + vat[i]) = vst[i];
   };
-  fetch_page(start_of(0));
-  fetch_tile(start_of(0));
-  if (ntile > 1) fetch_page(start_of(1));
+  fetch_page(start_of(it0));
+  fetch_tile(start_of(it0));
+  if (it0 + 1 < itn) fetch_page(start_of(it0 + 1));
 
   // Q^T: 8 entries of the lane's query per step of 16; a negative scale turns the query's sign
   const uint32_t flip = a.scale < 0.f ? 0x80008000u : 0u;
@@ -175,7 +194,8 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
     }
   }
   // m in log2 units; l is the lane's share of the sum: the sink's 1 goes to the lower half
-  float m = a.sink ? a.sink[head] * 1.4426950408889634f : -INFINITY, l = (a.sink && hi == 0) ? 1.f : 0.f;
+  const bool sunk = a.sink && stretch == 0;
+  float m = sunk ? a.sink[head] * 1.4426950408889634f : -INFINITY, l = (sunk && hi == 0) ? 1.f : 0.f;
   f16_t o[DT];
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) o[dt] = f16_t{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -183,12 +203,12 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
   // the lane's corner of a transposing read: its 16-lane group turns 4 keys x 16 values
   const int trow = 4 * hi + ((lane & 15) >> 2), tcol = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
 
-  put_tile(lds[0]);
-  for (int it = 0; it < ntile; ++it) {
+  put_tile(lds[it0 & 1]);
+  for (int it = it0; it < itn; ++it) {
     __syncthreads();  // this tile is whole, and nobody reads the other buffer any more
-    if (it + 1 < ntile) {
+    if (it + 1 < itn) {
       fetch_tile(start_of(it + 1));
-      if (it + 2 < ntile) fetch_page(start_of(it + 2));
+      if (it + 2 < itn) fetch_page(start_of(it + 2));
     }
     const int k0 = start_of(it);
     const bf16_t* kl = lds[it & 1];
@@ -266,10 +286,24 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
         }
       }
     }
-    if (it + 1 < ntile) put_tile(lds[(it + 1) & 1]);
+    if (it + 1 < itn) put_tile(lds[(it + 1) & 1]);
   }
   l = across(l, true);
   if (!qok) return;
+  if constexpr (SPLIT) {
+    if (hi == 0) {
+      pp[0] = m;
+      pp[1] = l;
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        if (32 * dt + 8 * b < dv)
+          *reinterpret_cast<float4*>(pp + 4 + 32 * dt + 8 * b + 4 * hi) =
+              make_float4(o[dt][4 * b], o[dt][4 * b + 1], o[dt][4 * b + 2], o[dt][4 * b + 3]);
+    return;
+  }
   const float inv = 1.f / l;
   bf16_t* op = a.out + static_cast<long>(row0 + qi) * (a.H * dv) + head * dv + 4 * hi;
 #pragma unroll
@@ -291,12 +325,42 @@ bool launch_chunk_attention(const ChunkArgs& a, int max_q, hipStream_t st) {
   const bool paged = a.kx == nullptr;
   if (a.dk % 16 || a.dv % 16 || a.dv > 128 || a.dk > (paged ? 128 : 192) || (!paged && (a.dn % 8 || a.dn > a.dk || a.G != a.H)))
     return false;
-  const dim3 grid(a.G, (static_cast<long>(max_q) * (a.H / a.G) + 127) / 128, a.S), block(256);
-  if (!paged) hipLaunchKernelGGL((chunk_attention_kernel<192, 128, 32, false>), grid, block, 0, st, a);
-  else if (a.dk <= 64 && a.dv <= 64) hipLaunchKernelGGL((chunk_attention_kernel<64, 64, 64, true>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((chunk_attention_kernel<128, 128, 32, true>), grid, block, 0, st, a);
+  const int n = a.nsplit > 1 ? a.nsplit : 1;
+  const dim3 grid(a.G, (static_cast<long>(max_q) * (a.H / a.G) + 127) / 128, a.S * n), block(256);
+  if (grid.z > 65535u) return false;
+#define MIX_CHUNK(...)                                                                                                       \
+  do {                                                                                                                       \
+    if (n > 1) hipLaunchKernelGGL((chunk_attention_kernel<__VA_ARGS__, true>), grid, block, 0, st, a);                       \
+    else hipLaunchKernelGGL((chunk_attention_kernel<__VA_ARGS__, false>), grid, block, 0, st, a);                            \
+  } while (0)
+  if (!paged) MIX_CHUNK(192, 128, 32, false);
+  else if (a.dk <= 64 && a.dv <= 64) MIX_CHUNK(64, 64, 64, true);
+  else MIX_CHUNK(128, 128, 32, true);
+#undef MIX_CHUNK
   MXS_CHECK_LAUNCH();
-  return true;
+  return n == 1 || launch_attention_combine(a.out, a.part, static_cast<long>(a.rows) * a.H, n, a.dv, st);
+}
+
+// Stretches pay where the longest walk counts and not the chip: a key costs a walk some 0.022 us (heads of 64; 0.04 with 128
+// entries), a stretch's records their bytes twice at 2 TB/s, the merge 6 us.  Whole against split, 32 heads of 64 over 8:
+// 64 rows behind 2,000 keys 49.7 / 21.6 us, 512 rows behind 2,000 62.3 / 44.7, behind 1,000 39.6 / 37.6; 1,024 rows with
+// nothing behind them 29.1 / 47.2 (two stretches, not chosen); 16 heads of 128 over 4:
+// 512 rows behind 2,000 105 / 49.  Up to about
+// two workgroups a unit, stretches of 512 keys or more.
+int chunk_attention_splits(long rows, int S, int H, int G, int dk, int dv, long span) {
+  const long tiles = G * (rows * (H / G) / 128 + S);
+  if (tiles == 0 || span < 1024) return 1;
+  int best = 1;
+  double gain = 0.;
+  for (int n = 2; n <= 4 && n * tiles <= 1024 && 512L * n <= span && S * n <= 65535; ++n) {
+    const double walk = static_cast<double>(span) * (dk + dv <= 128 ? 0.022 : 0.04);
+    const double g = walk * (1. - 1. / n) - 2. * 4. * (dv + 4) * rows * H * n / 2e6 - 6.;
+    if (g > gain) {
+      gain = g;
+      best = n;
+    }
+  }
+  return best;
 }
 
 // One workgroup: the sequences' row counts summed 256 at a time.

@@ -274,13 +274,16 @@ bool launch_window_attention(void* out, const void* q, long q_stride, const void
   a.bt_stride = bt_stride;
   a.koff = koff;
   a.voff = voff;
+  a.rows = rows;
+  a.nsplit = part ? nsplit : 1;
+  a.part = part;
   const bool pieces = bf && dk <= 128 && dv <= 128 && koff % 8 == 0 && voff % 8 == 0 && block_stride % 8 == 0;
   if (pieces && vs == dv && max_q >= 16 && bs == 16 && dk % 16 == 0 && dv % 16 == 0 && q_stride % 4 == 0 &&
       reinterpret_cast<uintptr_t>(q) % 8 == 0)
     return launch_chunk_attention(a, max_q, st);
   if (pieces && dk % 8 == 0 && dv % 8 == 0 && vs % 8 == 0 && (bs & (bs - 1)) == 0 && q_stride % 8 == 0 &&
       reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(cache) % 16 == 0) {
-    launch_row_attention(a, rows, bs, vs, part ? nsplit : 1, part, st);
+    launch_row_attention(a, rows, bs, vs, a.nsplit, part, st);
     MXS_CHECK_LAUNCH();
     return true;
   }

@@ -146,7 +146,8 @@ class WindowAttention(Mixer):
         seqmix.kv_write(ctx.cache, k, v, md.slot_mapping, koff, voff, self.kv_heads, self.dk, self.dv, ctx.block_size)
         o = seqmix.window_attention(q, ctx.cache, md.block_tables, md.query_start_loc, md.seq_lens, koff, voff,
                                     self.heads, self.kv_heads, self.dk, self.dv, ctx.block_size, self.scale,
-                                    self.window, self.keep_first, md.max_query_len)
+                                    self.window, self.keep_first, md.max_query_len,
+                                    max_seq_len=getattr(md, "max_seq_len", 0))
         return ops.linear(o, w[self.p + "o"])
 
 
@@ -368,7 +369,7 @@ class RotaryAttention(Mixer):
                               ctx.eps, self.v_freqs)
         o = seqmix.window_attention(q, ctx.cache, md.block_tables, md.query_start_loc, md.seq_lens, koff, voff,
                                     self.heads, self.kv_heads, self.dk, self.dv, ctx.block_size, self.scale, 0, 0,
-                                    md.max_query_len, sink=w.get(p + "sink"))
+                                    md.max_query_len, sink=w.get(p + "sink"), max_seq_len=getattr(md, "max_seq_len", 0))
         if not self.rotate_values and out is None and out_scale == 1.0:
             return o
         if out is None:
@@ -631,7 +632,8 @@ class LatentAttention(Mixer):
         qc = q[nd:]
         seqmix.rope_half_into(qc, qc, md.positions[nd:], H, dq, self.dn, dq, self.dn, self.freqs, self.split_pairs, self.mag)
         if seqmix.expanded_attention(qc, kv, rows, base, ctx.chunk_rows(), md.seq_lens[nd:], H, self.dn, self.dr, self.vd,
-                                     self.scale, md.max_query_len, w.get(p + "sink"), self.window, o[nd:]) is None:
+                                     self.scale, md.max_query_len, w.get(p + "sink"), self.window, o[nd:],
+                                     getattr(md, "max_seq_len", 0)) is None:
             raise RuntimeError(f"{p}: no kernel for heads of {self.dn} + {self.dr} / {self.vd} entries")  # q is turned already
         return True
 

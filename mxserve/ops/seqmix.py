@@ -404,7 +404,8 @@ def window_attention(q: torch.Tensor, cache: torch.Tensor, block_tables: torch.T
     holds exp(sink[h]), a key without a value whose score is not scaled.  v_stride (elements, 0: dv): the
     distance between two tokens' value rows, for values that are a slice of a wider cached row (then
     num_kv_heads is 1 and voff points at the slice inside the first row).  max_query_len: the longest chunk of the step (host
-    int); from 16 rows a bf16 step with head sizes that are multiples of 16 runs the MFMA kernel.
+    int); from 16 rows a bf16 step with head sizes that are multiples of 16 runs the MFMA kernel.  max_seq_len (host int,
+    0: not known): a bound of the keys, by which long walks of few chunks are split over workgroups.
     talk (fp32 [H, H]): the heads' scaled scores of a (query, key) pair are mixed before the softmax,
     score_h <- sum_g talk[h, g] score_g (the mask and the sink act on the mixed scores); a workgroup then
     serves all heads of its rows, and a bf16 step of few rows splits every row's keys over several
@@ -432,7 +433,7 @@ def window_attention(q: torch.Tensor, cache: torch.Tensor, block_tables: torch.T
         out = torch.empty(T, num_heads * dv, dtype=q.dtype, device=q.device)
         ext().window_attention(out, q, cache, block_tables, qsl, seq_lens, int(koff), int(voff), num_heads,
                                num_kv_heads, dk, dv, block_size, float(scale), int(window), int(keep_first),
-                               int(max_query_len), sink, int(v_stride))
+                               int(max_query_len), sink, int(v_stride), int(max_seq_len))
         return out
     out = torch.zeros(T, num_heads, dv, dtype=torch.float32)
     kc = cache[:, koff:koff + num_kv_heads * block_size * dk].view(-1, num_kv_heads, block_size, dk)
@@ -1244,18 +1245,20 @@ def latent_rows(cache: torch.Tensor, block_tables: torch.Tensor, base: torch.Ten
 
 def expanded_attention(q: torch.Tensor, kv: torch.Tensor, rows: torch.Tensor, base: torch.Tensor, qsl: torch.Tensor,
                        seq_lens: torch.Tensor, num_heads: int, dn: int, dr: int, dv: int, scale: float, max_query_len: int,
-                       sink: Optional[torch.Tensor] = None, window: int = 0,
-                       out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+                       sink: Optional[torch.Tensor] = None, window: int = 0, out: Optional[torch.Tensor] = None,
+                       max_seq_len: int = 0) -> Optional[torch.Tensor]:
     """Causal softmax attention of chunks over keys and values that every head expanded from gathered latent rows.
     q [T, H*(dn + dr)], kv [n, H*dn + H*dv]: the heads' plain key parts, then their values; the last dr entries of `rows`
     [n, rank + dr] are the key part that all heads share.  Row of key position j of sequence s: base[s] + j.  sink, window
-    as in latent_attention.  -> [T, H*dv] (in `out` if given); None: head sizes that the kernel does not hold."""
+    as in latent_attention, max_seq_len as in window_attention.  -> [T, H*dv] (in `out` if given); None: head sizes that the
+    kernel does not hold."""
     T, H, rank = q.shape[0], num_heads, rows.shape[1] - dr
     if out is None:
         out = torch.empty(T, H * dv, dtype=q.dtype, device=q.device)
     if _gpu(q):
         ok = q.dtype == torch.bfloat16 and ext().expanded_attention(out, q, kv, rows, base, qsl, seq_lens, H, dn, dr, dv, rank,
-                                                                    float(scale), int(max_query_len), sink, int(window))
+                                                                    float(scale), int(max_query_len), sink, int(window),
+                                                                    int(max_seq_len))
         return out if ok else None
     ql, sl, bl = qsl.tolist(), seq_lens.tolist(), base.tolist()
     for s in range(len(sl)):
