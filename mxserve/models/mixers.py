@@ -73,16 +73,16 @@ class StepContext:
             t = self.tables[key] = seqmix.rotary_table(self.md.positions, freqs, mag)
         return t
 
-    def expansion(self, window: int) -> Optional[tuple]:
+    def expansion(self, window: int, heads: int) -> Optional[tuple]:
         """(base, offs, rows): where the latent rows that this step's chunks see lie when they are gathered for every head to
         expand its own keys and values from them; None when the chunks are too short for that to pay, or their lengths are
         not known here."""
-        key = ("expansion", window)
+        key = ("expansion", window, heads)
         if key not in self.tables:
-            self.tables[key] = self._plan_expansion(window)
+            self.tables[key] = self._plan_expansion(window, heads)
         return self.tables[key]
 
-    def _plan_expansion(self, window: int) -> Optional[tuple]:
+    def _plan_expansion(self, window: int, heads: int) -> Optional[tuple]:
         md = self.md
         chunks, nd = getattr(md, "chunks", None), getattr(md, "num_decodes", 0)
         if not chunks or not md.seq_lens.is_cuda or len(chunks) + nd != md.seq_lens.numel():
@@ -92,7 +92,7 @@ class StepContext:
             first = max(past - window + 1, 0) // 16 * 16 if window > 0 else 0
             rows += past + n - first
             pairs += n * min(past + (n + 1) // 2, window if window > 0 else 1 << 30)
-        if pairs < EXPAND_MIN_QUERIES * rows:
+        if pairs < EXPAND_MIN_QUERIES * rows or pairs * heads < EXPAND_MIN_PAIRS:
             return None
         return seqmix.latent_plan(self.chunk_rows(), md.seq_lens[nd:], window) + (rows,)
 
@@ -107,7 +107,10 @@ class StepContext:
 # 2 * (dim + rot_dim + vdim) instead of the folded form's 2 * (2 rank + rot_dim) (128 + 64, 128, rank 512: 262,144 against
 # 1,536 saved, so from 170 queries on by operations alone); the folded form runs them at a third of the rate as well.  4,096 new
 # tokens, 16 heads of these sizes: 1,142 + 50 us folded (attention, two batched products), 217 + 32 us expanded.
+# It also takes six launches more in a layer (both forms run where single tokens stand beside chunks), which the host pays for
+# in a small step: below this many (query, key, head) triples the folded form's attention is under 70 us (8.5 ps a triple).
 EXPAND_MIN_QUERIES = 64
+EXPAND_MIN_PAIRS = 8 << 20
 EXPAND_MAX_BYTES = 1 << 30  # expanded keys and values of a layer; steps with more stay on the folded form
 
 
@@ -611,8 +614,10 @@ class LatentAttention(Mixer):
         nd = T
         if h.dtype == torch.bfloat16 and self._expand(q, o, w, ctx, koff):
             nd = md.num_decodes
-        if nd:
-            self._fold(q[:nd], o[:nd], w, ctx, koff, nd < T)
+        if nd == T:
+            self._fold(q, o, w, ctx, koff, False)
+        elif nd:
+            self._fold(q[:nd], o[:nd], w, ctx, koff, True)
         return ops.linear(o, w[p + "o"])
 
     def _expand(self, q: torch.Tensor, o: torch.Tensor, w: dict, ctx: StepContext, koff: int) -> bool:
@@ -623,7 +628,7 @@ class LatentAttention(Mixer):
         plan = None
         if dq <= 192 and dq % 16 == 0 and self.vd <= 128 and self.vd % 16 == 0 and self.dn % 8 == 0 and self.dr % 8 == 0 and \
                 self.rank % 8 == 0 and koff % 8 == 0 and ctx.cache.shape[1] % 8 == 0 and ctx.block_size == 16:
-            plan = ctx.expansion(self.window)
+            plan = ctx.expansion(self.window, H)
         if plan is None or 2 * plan[2] * H * (self.dn + self.vd) > EXPAND_MAX_BYTES:
             return False
         base, offs, n = plan
@@ -642,14 +647,14 @@ class LatentAttention(Mixer):
         query and W_uv applied to the weighted sum."""
         md, p, H = ctx.md, self.p, self.heads
         T, dq_, dk = q.shape[0], self.dn + self.dr, self.dk
-        bt, qsl, lens, mq = md.block_tables, md.query_start_loc, md.seq_lens, md.max_query_len
+        bt, qsl, lens, pos, mq = md.block_tables, md.query_start_loc, md.seq_lens, md.positions, md.max_query_len
         if singles:
-            bt, qsl, lens, mq = bt[:T], qsl[:T + 1], lens[:T], 1
+            bt, qsl, lens, pos, mq = bt[:T], qsl[:T + 1], lens[:T], pos[:T], 1
         qf = torch.empty(T, H * dk, dtype=q.dtype, device=q.device)
         # the plain part through W_uk^T, head by head, straight into its columns of the folded query
         torch.bmm(q.view(T, H, dq_)[:, :, :self.dn].transpose(0, 1), w[p + "uk"],
                   out=qf.view(T, H, dk)[:, :, :self.rank].transpose(0, 1))
-        seqmix.rope_half_into(qf, q, md.positions[:T], H, dq_, self.dn, dk, self.rank, self.freqs, self.split_pairs, self.mag)
+        seqmix.rope_half_into(qf, q, pos, H, dq_, self.dn, dk, self.rank, self.freqs, self.split_pairs, self.mag)
         lat = seqmix.latent_attention(qf, ctx.cache, bt, qsl, lens, koff, H, dk, self.rank, ctx.block_size, self.scale, mq,
                                       getattr(md, "max_seq_len", 0), sink=w.get(p + "sink"), window=self.window)
         torch.bmm(lat.view(T, H, self.rank).transpose(0, 1), w[p + "uv"], out=o.view(T, H, self.vd).transpose(0, 1))

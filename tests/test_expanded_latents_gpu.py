@@ -68,6 +68,7 @@ def test_mixer_expands_and_folds(gpu, monkeypatch, window, singles):
     """A step of chunks (and single tokens before them): what the mixer gives with the chunks' lengths known and unknown,
     both against the formulas in 64 bits; the expanded way is no further off."""
     monkeypatch.setattr(mixers, "EXPAND_MIN_QUERIES", 16)  # chunks of this size fold when left to themselves
+    monkeypatch.setattr(mixers, "EXPAND_MIN_PAIRS", 0)
     W, H, dn, dr, vd, rank, qr = 256, 4, 128, 64, 128, 128, 192
     rot = {"dims": dr, "base": 10000.0}
     m = LatentAttention("", W, H, dn, dr, vd, rank, qr, 192 ** -0.5, rot, window=window)
@@ -105,7 +106,7 @@ def test_mixer_expands_and_folds(gpu, monkeypatch, window, singles):
         ctx = StepContext(md=md, cache=c, state=None, block_size=16, eps=1e-5)
         y = h.to(gpu) @ w_in.T
         outs[way] = m.forward([y[:, :qr], y[:, qr:]], h.to(gpu), wg, ctx, 0, 0, 0).cpu().double()
-        assert (ctx.expansion(window) is not None) == (way == "expanded")
+        assert (ctx.expansion(window, H) is not None) == (way == "expanded")
     d = {k: t.double() for k, t in w.items()}
     f = torch.tensor([10000.0 ** (-2.0 * i / dr) for i in range(dr // 2)], dtype=torch.float64)
 
