@@ -89,7 +89,7 @@ __global__ void __launch_bounds__(256) window_attention_kernel(
 }
 
 
-// ---- Row form with 16-byte loads (single decoded tokens, short chunks): head sizes that are
+// ---- Row form with 16-byte loads (fp32, and bf16 heads that row_attention.hip does not hold): head sizes that are
 // multiples of 16 bytes.  Eight lanes share a key: each loads 16 bytes of every 128-byte stretch of
 // the key's row, so a wave's load instruction covers eight whole rows instead of 64 two-byte (or 64
 // scattered 16-byte) pieces; the score is summed over the eight lanes.  The value rows are read the
