@@ -17,6 +17,7 @@
 // 2-byte reads of V (the form that this one replaced), 139 us; window 1,024: 75 us; 16 heads of 128: 192 us.  Keys of 128 + 64 and values of 128 expanded from latent rows of 576, 16 heads,
 // 4,096 rows: 217 us and 50 us for gathering and expanding, against 1,142 us over the rows themselves with folded queries.
 #include "chunk_attention.h"
+#include "chunk_walk.h"
 #include "mix_common.h"
 
 #include <algorithm>
@@ -103,11 +104,9 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
     __syncthreads();
   }
 
-  // tiles: those of the kept first tokens below the window, then from the window's first to the diagonal
-  const int t0 = (a.window > 0 ? max(past + first / R - a.window + 1, 0) : 0) / KT;
-  const int nA = a.window > 0 ? min((a.keep + KT - 1) / KT, t0) : 0;
-  const int ntile = nA + glast / KT - t0 + 1;
-  auto start_of = [&](int it) { return (it < nA ? it : t0 + it - nA) * KT; };
+  const ChunkWalk walk = chunk_walk(past + first / R, glast, a.window, a.keep, KT);
+  const int ntile = walk.ntile;
+  auto start_of = [&](int it) { return walk.start(it); };
 
   // this workgroup's tiles: all, or its stretch of a long walk (short walks are the first stretch's alone)
   int it0 = 0, itn = ntile;
@@ -128,7 +127,7 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
 
   const int* bt = PAGED ? a.block_tables + static_cast<long>(s) * a.bt_stride : nullptr;
   const int lastpage = PAGED ? min(glast >> 4, a.bt_stride - 1) : 0;
-  const int dense0 = PAGED ? 0 : a.base[s];
+  const int dense0 = PAGED ? 0 : a.base[s], low0 = PAGED ? 0 : first_gathered(past, a.window);
   const int kmax = PAGED ? glast : min(glast, a.nrows - 1 - dense0);  // the last key that may be read
   int page = 0;  // of the tile to be fetched next
   auto fetch_page = [&](int k0) {
@@ -148,8 +147,8 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
       vb = a.vx + r * a.x_stride + g * dv;
       rb = a.kr + r * a.r_stride;
     }
-    // keys past the last one anybody here sees may hold anything: zeros
-    const int left = kmax - key0;
+    // keys past the last one anybody here sees may hold anything, and there are no rows before the first gathered one: zeros
+    const int left = PAGED ? kmax - key0 : gathered_left(key0, low0, kmax);
 #pragma unroll
     for (int i = 0; i < NK; ++i) {
       kst[i] = make_uint4(0, 0, 0, 0);
@@ -374,7 +373,7 @@ __global__ void __launch_bounds__(256) latent_plan_kernel(int* __restrict__ base
     int n = 0, firstkey = 0;
     if (s < S) {
       const int qlen = qsl[s + 1] - qsl[s], past = max(seq_lens[s] - qlen, 0);
-      firstkey = window > 0 ? max(past - window + 1, 0) & ~15 : 0;
+      firstkey = first_gathered(past, window);
       n = qlen > 0 ? past + qlen - firstkey : 0;
     }
     sum[threadIdx.x] = n;

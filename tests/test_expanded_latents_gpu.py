@@ -62,6 +62,38 @@ def test_gathered_rows_and_their_attention(gpu, H, dn, dr, dv, rank, chunks, win
             assert float(err.max()) <= 2.0 ** -13 * float(kv.float().abs().max()), (s, float(err.max()))
 
 
+@pytest.mark.parametrize("oldest", [0, 15, 16, 31, 32, 47, 2048, 2063])
+@pytest.mark.parametrize("window,new", [(40, 130), (17, 20), (1024, 300)])
+def test_windowed_rows_between_others(gpu, oldest, window, new):
+    """The rows around a sequence's own are no numbers, before the first sequence and between two: a tile that begins a page
+    before the first gathered row takes nothing from there."""
+    H, dn, dr, dv, rank = 2, 128, 64, 128, 64
+    g = torch.Generator().manual_seed(oldest + window)
+    past = oldest + window - 1  # the first query's oldest key is `oldest`
+    chunks = [(past, new), (0, 16), (past, new)]
+    qsl = torch.tensor([0] + [n for _, n in chunks]).cumsum(0).int()
+    lens = torch.tensor([p + n for p, n in chunks], dtype=torch.int32)
+    base, offs = seqmix.latent_plan(qsl.to(gpu), lens.to(gpu), window)
+    off = offs.tolist()
+    q = torch.randn(int(qsl[-1]), H * (dn + dr), generator=g).bfloat16()
+    kv, rows = (torch.full((off[-1] + 64, n), float("nan"), dtype=torch.bfloat16) for n in (H * (dn + dv), rank + dr))
+    for a, e in ((off[0], off[1]), (off[2], off[3])):  # the second sequence's rows are no numbers either
+        kv[32 + a:32 + e] = torch.randn(e - a, kv.shape[1], generator=g).bfloat16()
+        rows[32 + a:32 + e] = torch.randn(e - a, rows.shape[1], generator=g).bfloat16()
+    inner = slice(32, 32 + off[-1])
+    sink, scale = torch.randn(H, generator=g), (dn + dr) ** -0.5
+    got = seqmix.expanded_attention(q.to(gpu), kv.to(gpu)[inner], rows.to(gpu)[inner], base, qsl.to(gpu), lens.to(gpu), H, dn, dr, dv,
+                                    scale, new, sink.to(gpu), window, max_seq_len=past + new).cpu().double()
+    kv, rows = kv[inner], rows[inner]
+    for s in (0, 2):
+        a, e, r = int(qsl[s]), int(qsl[s + 1]), slice(off[s], off[s + 1])
+        K = torch.cat([kv[r, :H * dn].view(-1, H, dn), rows[r, rank:].unsqueeze(1).expand(-1, H, -1)], -1).double()
+        want = softmax_mix(q[a:e].double().view(-1, H, dn + dr), K, kv[r, H * dn:].view(-1, H, dv).double(), past, scale, sink, window,
+                           off[s] - int(base[s])).reshape(e - a, -1)
+        err = (got[a:e] - want).abs() - 2.0 ** -8 * want.abs()  # as above
+        assert float(err.max()) <= 2.0 ** -13 * float(kv[r].float().abs().max()), (s, float(err.max()))
+
+
 @pytest.mark.parametrize("window", [0, 50])
 @pytest.mark.parametrize("singles", [0, 3])
 def test_mixer_expands_and_folds(gpu, monkeypatch, window, singles):
