@@ -27,6 +27,7 @@ from ..config import EngineArgs
 from ..models.config import ModelConfig
 from ..models.llama import AttnMetadata, build_model
 from ..models.weights import load_weights
+from ..ops.decode_gemm import Workspace, using
 from ..parallel.comm import (collectives_capturable, collectives_local, get_tp, setup_meta_ring, tp_barrier,
                              tp_broadcast_object)
 from ..parallel.custom_allreduce import CollectiveFault
@@ -188,6 +189,7 @@ class ModelRunner:
             self._err_pinned = [torch.zeros(8, dtype=torch.int32, pin_memory=True) for _ in range(2)]
             self._err_events = [torch.cuda.Event(), torch.cuda.Event()]
         self.graphs: dict[int, tuple] = {}
+        self.gemm_ws = Workspace()  # this engine's own: its graphs hold the addresses
         if get_tp().tp_size > 1:  # every rank's start-up work is done before the first collective
             tp_barrier()
         if self.is_gpu and not args.enforce_eager:
@@ -501,7 +503,8 @@ class ModelRunner:
             g.replay()
             self._logits = logits
             return out[:meta["S"]]
-        return self._forward_eager(meta, sample=bool(meta["sample_rows"]))
+        with using(self.gemm_ws):
+            return self._forward_eager(meta, sample=bool(meta["sample_rows"]))
 
     def follower_loop(self) -> None:
         """TP ranks > 0: mirror the driver's steps until it broadcasts shutdown."""
@@ -646,9 +649,10 @@ class ModelRunner:
             log.warning("no decode bucket has graph-capturable collectives; decode runs eagerly")
             return
         # a model without tunable projections (its tunable_shapes() is empty) runs the library's choice
-        if tune and (not hasattr(m, "tunable_shapes") or m.tunable_shapes()):
-            self._tune_gemms(buckets)
-        self._capture(buckets)
+        with using(self.gemm_ws):
+            if tune and (not hasattr(m, "tunable_shapes") or m.tunable_shapes()):
+                self._tune_gemms(buckets)
+            self._capture(buckets)
 
     def _tune_gemms(self, buckets: list) -> None:
         m = self.model
@@ -759,7 +763,7 @@ class ModelRunner:
             torch.cuda.synchronize(self.device)
         self.graphs.clear()
         self._logits = None
-        for name in ("kv_cache", "state", "model", "bt_dev", "last_tok", "hist", "_pen_counts", "buf"):
+        for name in ("kv_cache", "state", "model", "bt_dev", "last_tok", "hist", "_pen_counts", "buf", "gemm_ws"):
             setattr(self, name, None)
 
     def kv_stats(self) -> dict:

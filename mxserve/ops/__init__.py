@@ -203,9 +203,6 @@ def _run_mplan(x: torch.Tensor, w: torch.Tensor, plan: list) -> torch.Tensor:
     return y
 
 
-_PG_PART: dict = {}
-
-
 def _decode_max_m() -> int:
     from .decode_gemm import MAX_M
     return MAX_M
@@ -222,10 +219,10 @@ def prefill_gemm(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, cfg: tuple
     bm, sk = cfg
     part = None
     if sk > 1:
-        need = sk * x.shape[0] * w.shape[0]
-        part = _PG_PART.get(x.device)
-        if part is None or part.numel() < need:
-            part = _PG_PART[x.device] = torch.empty(need, dtype=torch.float32, device=x.device)
+        from .decode_gemm import workspace
+        part = workspace().slabs(sk * x.shape[0] * w.shape[0], x.device)
+        if part is None:
+            return False
     return bool(ext().prefill_gemm(out, x, w, part, bm, sk))
 
 

@@ -16,6 +16,7 @@ import bisect
 import json
 import logging
 import os
+import threading
 import time
 from typing import Optional
 
@@ -176,13 +177,85 @@ def _candidates_mf(M: int, N: int, K: int, epi: int, mf: int) -> list[tuple]:
     return out
 
 
+class Workspace:
+    """What the split-K products of one engine leave between their kernels.  A captured graph holds the addresses, so an
+    engine's graphs and its eager steps run on a workspace of their own (`using`), which lives as long as the engine, and a
+    slab that is outgrown stays: each is at least twice the one before, so those kept are smaller than the last."""
+
+    def __init__(self):
+        self.part: Optional[torch.Tensor] = None  # fp32 split-K slabs
+        self.cnt: Optional[torch.Tensor] = None  # mt kernel tile counters (in-launch split-K reduce)
+        self.outgrown: list = []
+
+    def slabs(self, need: int, device) -> Optional[torch.Tensor]:
+        """The slabs, at least `need` floats; None where a capture is under way and they would have to grow."""
+        p = self.part
+        if p is not None and p.numel() >= need and p.device == device:
+            return p
+        if _capturing():
+            return None
+        if p is not None:
+            self.outgrown.append(p)
+            need = max(need, 2 * p.numel())
+        self.part = torch.empty(need, dtype=torch.float32, device=device)
+        return self.part
+
+    def counters(self, device) -> Optional[torch.Tensor]:
+        if self.cnt is None or self.cnt.device != device:
+            if _capturing():
+                return None
+            if self.cnt is not None:
+                self.outgrown.append(self.cnt)
+            self.cnt = torch.zeros(MT_COUNTERS, dtype=torch.int32, device=device)
+        return self.cnt
+
+
+def _capturing() -> bool:
+    return torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
+
+
+_THREAD = threading.local()
+_SHARED = Workspace()  # products outside of an engine
+
+
+def workspace() -> Workspace:
+    """The calling thread's workspace."""
+    return getattr(_THREAD, "workspace", None) or _SHARED
+
+
+class using:
+    """with using(ws): this thread's products run on ws."""
+
+    def __init__(self, ws: Workspace):
+        self.ws = ws
+
+    def __enter__(self) -> Workspace:
+        self.before = getattr(_THREAD, "workspace", None)
+        _THREAD.workspace = self.ws
+        return self.ws
+
+    def __exit__(self, *exc) -> None:
+        _THREAD.workspace = self.before
+
+
 class DecodeGemmTable:
     def __init__(self):
         self.entries: dict[tuple, list] = {}  # (N, K, epi) -> sorted [(M bucket, cfg or None)]
-        self.part: Optional[torch.Tensor] = None  # fp32 split-K workspace (stable for graphs)
-        self.cnt: Optional[torch.Tensor] = None  # mt kernel tile counters (in-launch split-K reduce)
         self.report: list = []
         self.store_stats: dict = {}
+
+    # the calling thread's workspace, where the caller's epilogue kernel finds the slabs
+    @property
+    def part(self) -> Optional[torch.Tensor]:
+        return workspace().part
+
+    @part.setter
+    def part(self, t: Optional[torch.Tensor]) -> None:
+        workspace().part = t
+
+    @property
+    def cnt(self) -> Optional[torch.Tensor]:
+        return workspace().cnt
 
     def lookup(self, M: int, N: int, K: int, epi: int) -> Optional[tuple]:
         if MODE == "off" or M > MAX_M:
@@ -210,8 +283,8 @@ class DecodeGemmTable:
 
     def run(self, out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, cfg: tuple, epi: int,
             reduce: bool = True) -> bool:
-        """reduce=False (split-K configurations only): leave the fp32 slabs [sk][M][N] in self.part for
-        the caller's epilogue kernel (ops.linear_add_rms_norm)."""
+        """reduce=False (split-K configurations only): leave the fp32 slabs [sk][M][N] in `part`, the thread's
+        workspace, for the caller's epilogue kernel (ops.linear_add_rms_norm)."""
         from . import ext
         if cfg[0] == "pf":
             from . import gemm_pf
@@ -222,12 +295,9 @@ class DecodeGemmTable:
                 return False  # SwiGLU applies in the reduce
             part = None
             if kg > 1:
-                need = kg * x.shape[0] * w.shape[0]
-                if self.part is None or self.part.numel() < need:
-                    if torch.cuda.is_current_stream_capturing():
-                        return False
-                    self.part = torch.empty(need, dtype=torch.float32, device=x.device)
-                part = self.part
+                part = workspace().slabs(kg * x.shape[0] * w.shape[0], x.device)
+                if part is None:
+                    return False
             return bool(ext().gemv_stream(out, x, w, part, int(cfg[1]), int(cfg[2]), int(epi), kg, reduce))
         if cfg[0] == "sk":
             groups = w.shape[1] // (4 * int(cfg[1]))
@@ -235,12 +305,9 @@ class DecodeGemmTable:
                 return False
             part = None
             if groups > 1 or epi:
-                need = groups * x.shape[0] * w.shape[0]
-                if self.part is None or self.part.numel() < need:
-                    if torch.cuda.is_current_stream_capturing():
-                        return False
-                    self.part = torch.empty(need, dtype=torch.float32, device=x.device)
-                part = self.part
+                part = workspace().slabs(groups * x.shape[0] * w.shape[0], x.device)
+                if part is None:
+                    return False
             return bool(ext().skinny_gemm(out, x, w, part, int(cfg[1]), reduce, int(epi)))
         mt = cfg[0] == "mt"
         if mt:
@@ -251,19 +318,16 @@ class DecodeGemmTable:
             lu = cfg[4] if len(cfg) > 4 else 0
         part = None
         if sk > 1:
-            need = sk * x.shape[0] * w.shape[0]
-            if self.part is None or self.part.numel() < need:
-                if torch.cuda.is_current_stream_capturing():
-                    return False  # never allocate inside a capture (tune() sizes it beforehand)
-                self.part = torch.empty(need, dtype=torch.float32, device=x.device)
-            part = self.part
+            part = workspace().slabs(sk * x.shape[0] * w.shape[0], x.device)
+            if part is None:
+                return False  # never allocate inside a capture (tune() sizes it beforehand)
         if mt:
-            if sk > 1 and (self.cnt is None or self.cnt.device != x.device):
-                if torch.cuda.is_current_stream_capturing():
+            cnt = None
+            if sk > 1 and MT_FUSED_REDUCE and reduce:
+                cnt = workspace().counters(x.device)
+                if cnt is None:
                     return False
-                self.cnt = torch.zeros(MT_COUNTERS, dtype=torch.int32, device=x.device)
-            return bool(ext().mt_gemm(out, x, w, part, wm, wn, mr, wnf, sk, epi,
-                                      self.cnt if MT_FUSED_REDUCE and reduce else None, order, reduce))
+            return bool(ext().mt_gemm(out, x, w, part, wm, wn, mr, wnf, sk, epi, cnt, order, reduce))
         return bool(ext().decode_gemm(out, x, w, part, mf, nf, wm, sk, epi, lu, reduce))
 
 
@@ -379,9 +443,7 @@ def tune(shapes: dict, buckets: list, device, dtype=torch.bfloat16) -> list:
         return []
     store = TunedStore("decode_gemm", device_tag(device))
     # workspace for the largest split-K any candidate may pick
-    need = max(max(SPLITS) * max(bks) * v[0].shape[0] for v in shapes.values())
-    TABLE.part = torch.empty(need, dtype=torch.float32, device=device)
-    TABLE.cnt = torch.zeros(MT_COUNTERS, dtype=torch.int32, device=device)
+    workspace().slabs(max(max(SPLITS) * max(bks) * v[0].shape[0] for v in shapes.values()), next(iter(shapes.values()))[0].device)
     rows = []
     for name, val in shapes.items():
         w, epi = val[0], val[1]
