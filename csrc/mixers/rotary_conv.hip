@@ -341,7 +341,7 @@ __global__ void __launch_bounds__(256) causal_conv_rows_kernel(T* __restrict__ o
   for (int r = 0; r < kConvRows; ++r) {
     const int t = t0 + r;
     if (t >= rows) break;
-    if (r > 0 && t == qsl[s + 1]) {
+    if (r > 0 && s + 1 < S && t == qsl[s + 1]) {  // rows past the last sequence go on as its own
       do ++s; while (s + 1 < S && qsl[s + 1] <= t);
       look_back(t);
     }

@@ -92,6 +92,27 @@ def test_convolution_rows(gpu, dt, C, taps, lens):
 
 
 @pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("taps", [2, 4])
+@pytest.mark.parametrize("lens", [[3], [5, 2], [4, 9, 0], [1, 1, 1]])
+@pytest.mark.parametrize("more", [1, 2, 7])
+def test_convolution_rows_past_the_last_sequence(gpu, dt, taps, lens, more):
+    """x holds more rows than the sequences have: those go on as the last sequence's, and no sequence behind it is looked up."""
+    C, T, S = 72, sum(lens) + more, len(lens)
+    g = torch.Generator().manual_seed(T)
+    x, w = torch.randn(T, C, generator=g).to(dt), torch.randn(taps, C, generator=g).to(dt)
+    state = torch.randn(S, (taps - 1) * C, generator=g)
+    rows = torch.arange(S, dtype=torch.int32)
+    qsl = torch.tensor([0] + lens).cumsum(0).int()
+    seq = torch.tensor([n + 9 for n in lens], dtype=torch.int32)
+    on = [t.to(gpu) for t in (rows, qsl, seq)]
+    got = seqmix.causal_conv(x.to(gpu), w.to(gpu), None, state.to(gpu), on[0], 0, on[1], on[2], True, max(max(lens), 2)).cpu()
+    longer = qsl.clone()
+    longer[S] = T
+    want = seqmix.causal_conv(x, w, None, state.clone(), rows, 0, longer, seq + torch.tensor([0] * (S - 1) + [more]), True, T)
+    torch.testing.assert_close(got.float(), want.float(), **tol(dt))
+
+
+@pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("N,groups,wn", [(16, 2, 16), (128, 16, 8), (384, 8, 48), (384, 3, 384), (2048, 16, 128), (4096, 8, 4096), (1024, 1, 1024),
                                          (4096, 1, 4096), (8192, 2, 8192), (6144, 2, 6144)])
 def test_gated_norm_rows(gpu, dt, N, groups, wn):
