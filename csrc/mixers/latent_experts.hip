@@ -61,9 +61,10 @@ __global__ void __launch_bounds__(256) latent_prep_kernel(
   }
 }
 
+// out may be x, its own columns (a thread reads a pair before it writes it): neither pointer is __restrict__.
 template <typename T>
 __global__ void __launch_bounds__(256) rope_half_into_kernel(
-    T* __restrict__ out, long out_stride, const T* __restrict__ x, long x_stride, const int64_t* __restrict__ positions,
+    T* out, long out_stride, const T* x, long x_stride, const int64_t* __restrict__ positions,
     int heads, int x_dim, int x_col, int out_dim, int out_col, const float* __restrict__ freqs, int nf, int split, float mag) {
   const long t = blockIdx.x;
   const float pos = static_cast<float>(positions[t]);

@@ -1160,7 +1160,8 @@ def rope_half_into(out: torch.Tensor, x: torch.Tensor, positions: torch.Tensor, 
                    out_dim: int, out_col: int, freqs: torch.Tensor, split_pairs: bool = True, mag: float = 1.0) -> None:
     """Per token and head: the 2n columns of x's head (x [T, heads*x_dim], from column x_col of the head)
     turned in the half-split layout (split_pairs False: as neighbouring pairs) by position * freqs[i] (cos and sin
-    times mag), written to columns out_col.. of the same head in out [T, heads*out_dim].  fp32 inside."""
+    times mag), written to columns out_col.. of the same head in out [T, heads*out_dim].  out may be x with the same
+    columns (turned in place).  fp32 inside."""
     n = freqs.numel()
     if _gpu(x):
         ext().rope_half_into(out, x, positions, int(heads), int(x_dim), int(x_col), int(out_dim), int(out_col), freqs,

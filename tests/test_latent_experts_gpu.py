@@ -72,3 +72,23 @@ def test_latent_attention_without_sink_and_fp32():
     got = seqmix.latent_attention(q.to(dev).bfloat16(), cache.to(dev).bfloat16(), bt.to(dev), qsl.to(dev), sl.to(dev), 8, 4,
                                   96, 64, 16, 0.2, 50, 50)
     assert (got.float().cpu() - want).abs().max().item() < 0.03
+
+
+@pytest.mark.parametrize("split", [True, False])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,dn,dr", [(1, 8, 2), (16, 128, 64), (40, 64, 128), (3, 16, 30)])
+def test_heads_turned_in_place(dt, split, heads, dn, dr):
+    """rope_half_into with out = x gives, in the turned columns, what it gives into another tensor, and leaves the others."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    g = torch.Generator().manual_seed(heads)
+    T, dim = 5, dn + dr
+    x = torch.randn(T, heads * dim, generator=g).to(dt).cuda()
+    pos = torch.tensor([0, 3, 4095, 17, 100000], device="cuda")
+    fr = (torch.rand(dr // 2, generator=g) * 0.01).cuda()
+    apart = x.clone()
+    seqmix.rope_half_into(apart, x, pos, heads, dim, dn, dim, dn, fr, split, 1.25)
+    inside = x.clone()
+    seqmix.rope_half_into(inside, inside, pos, heads, dim, dn, dim, dn, fr, split, 1.25)
+    assert torch.equal(inside, apart)
+    assert torch.equal(inside.view(T, heads, dim)[:, :, :dn], x.view(T, heads, dim)[:, :, :dn])
