@@ -167,9 +167,10 @@ struct MemRow {
 // 128k row) are collected and ranked against each other; a fuller bin is cut again.  Two passes over the row where a
 // bisection over value took 32, each with an exponential per logit: that was what a row's time went into, and a row is
 // one workgroup, so a step with few sampled rows waits for it (MI355X, 128,256 bf16 logits, 13 rows: 275 us; 32,000
-// fp32 logits, 64 rows: 177 us.  Now 82 us and 27 us).  Weights are 2^-32 fixed point summed in 64-bit integers (shares
-// are at most 1): the sums do not depend on the order of the LDS atomics, so a request's tokens stay reproducible, and
-// they are closer to the exact ones than fp32 sums.
+// fp32 logits, 64 rows: 177 us.  Now 82 us and 27 us).  Shares (at most 1) are 2^-46 fixed point, what 64-bit sums of
+// 2^17 of them hold, with a bit less for each doubling of the row beyond: the sums do not depend on the order of the LDS
+// atomics, so a request's tokens stay reproducible.  A share loses less than a step, a row 2^-29 of its sum, where an fp32
+// sum rounds at 2^-24 (one word of 32 bits a share, 2^-15 of a row: 2 us less of 60).
 constexpr int kSelBins = 2048, kSelList = 512;
 struct SelLds {
   unsigned long long hist[kSelBins];
@@ -180,16 +181,18 @@ struct SelLds {
   int n, bin;
 };
 
-// by_share: weight 2^32 exp2((x - mx) * invt2), target `goal` of the whole; otherwise weight 1, target goal itself.
+// by_share: weight 2^32 hscale exp2((x - mx) * invt2), target `goal` of the whole; otherwise weight 1, target goal itself.
 // lo <= hi finite; logits outside [lo, hi] have no weight.  -inf when even all of them stay below the target.
 template <class Row>
 __device__ __forceinline__ float select_threshold(Row& R, SelLds& L, float* sv, bool by_share, double goal, float mx,
-                                                  float invt2, float lo, float hi) {
+                                                  float invt2, float hscale, float lo, float hi) {
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   auto weight = [&](float x) -> unsigned long long {
-    return by_share ? static_cast<unsigned long long>(static_cast<uint32_t>(
-                          fmaf(__builtin_amdgcn_exp2f((x - mx) * invt2), 4294967040.f, 0.5f)))
-                    : 1ull;
+    if (!by_share) return 1ull;
+    const float a = __builtin_amdgcn_exp2f((x - mx) * invt2) * hscale;
+    const uint32_t up = static_cast<uint32_t>(a);  // both words are exact
+    const uint32_t low = static_cast<uint32_t>(__builtin_amdgcn_fractf(a) * 4294967296.f);
+    return static_cast<unsigned long long>(up) << 32 | low;
   };
   unsigned long long above = 0, target = 0;
   for (int level = 0; level < 8; ++level) {
@@ -316,10 +319,12 @@ __global__ void __launch_bounds__(1024) sample_kernel(int64_t* __restrict__ out,
     if (mx == INFINITY) {  // nothing below an infinite logit has a share
       thr = mx;
     } else if (mx > -INFINITY) {
+      // a share of 1 is 2^32 hscale; the row's shares together stay below 2^63
+      const float hscale = V <= 1 << 17 ? 16384.f : static_cast<float>(1u << max(__clz(V - 1) - 1, 0));
       for (int by_share = 0; by_share < 2; ++by_share) {
         if (by_share ? p < 1.f : k > 0 && k < V)
           thr = fmaxf(thr, select_threshold(R, L, sv, by_share != 0, by_share ? static_cast<double>(p) : static_cast<double>(k),
-                                            mx, invt2, by_share ? fmaxf(mn, mx - 88.f * t) : mn, mx));
+                                            mx, invt2, hscale, by_share ? fmaxf(mn, mx - 88.f * t) : mn, mx));
       }
     }
   }

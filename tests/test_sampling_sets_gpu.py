@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 def exact_set(row: torch.Tensor, t: float, k: int, p: float, slack: float) -> torch.Tensor:
     """The tokens that may be sampled, in 64 bits; slack widens (> 0) or narrows (< 0) the nucleus by that share, more
-    than the kernel's 2^-32 fixed-point shares and the rounding of their exponentials (2^-22 each) can move it."""
+    than the kernel's 2^-46 fixed-point shares (2^-29 of a row) and the rounding of their exponentials (2^-22 each, and
+    2^-24 of the exponent) can move it."""
     z = row.double()
     keep = torch.isfinite(z)
     if 0 < k < z.numel():
@@ -69,3 +70,27 @@ def test_sampled_tokens_are_the_sets_maxima(gpu, dtype, V, kind):
         # fp32 scores: two hardware logarithms of about 2^-22 relative error each, around values of up to |z| / t
         tol = 1e-5 * max(1.0, float(score[wide].abs().max()))
         assert float(score[got]) >= float(score[narrow].max()) - tol, (kind, V, cases[i])
+
+
+@pytest.mark.parametrize("V", [131072, 262144, 300007])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_many_small_shares_count(gpu, dtype, V):
+    """131,000 tokens of 2^-34 of the likeliest one's share are 8e-6 of the whole and move the border of a nucleus that ends
+    among the tokens before them.  The second token lies where the row's noise makes it the maximum, so that the sample tells."""
+    for seed in range(1000):
+        u = ref.uniform_noise(torch.tensor([seed]), torch.tensor([2]), V)[0].double()
+        noise = -torch.log(-torch.log(u))
+        if float(noise.max()) > 16.0:
+            break
+    mid, first = int(noise.argmax()), int(noise.argmin())
+    z = torch.full((V,), -34 * 0.6931471805599453)
+    others = [v for v in (7, 7777, 77777, 100003) if v not in (mid, first)]
+    z[others], z[mid], z[first] = -14.25, -13.75, 0.0
+    z = z.to(dtype)
+    share = torch.exp(z.double() - float(z[first]))
+    p = float((share[first] + 0.5 * share[mid]) / share.sum())  # half way into the second token: fp32 steps of p are 6e-8
+    assert abs(float(torch.tensor(p)) - p) < 0.1 * float(share[mid])
+    one = lambda x, t: torch.tensor([x], dtype=t, device=gpu)  # noqa: E731
+    got = ops.sample(z.view(1, V).to(gpu), one(1.0, torch.float32), one(p, torch.float32), one(0, torch.int32),
+                     one(seed, torch.int64), one(2, torch.int64))
+    assert int(got[0]) == mid
