@@ -14,6 +14,7 @@
 // 64, state 128, both passes: 720 us token by token on the vector units, 125 us
 // here, and with less error against 64 bits (2e-7 of y's norm against 5e-7 at half lives of a thousand tokens).
 #include <algorithm>
+#include <limits>
 
 #include "mix_common.h"
 #include "column_scan.h"
@@ -64,6 +65,12 @@ __device__ __forceinline__ b8_t col_perm(const bf16_t* p, int pitch) {
   return pair4(__builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(p)), __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(p + 8 * pitch)));
 }
 __device__ __forceinline__ f16_t mm(b8_t a, b8_t b, f16_t c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+typedef unsigned short u2_t __attribute__((ext_vector_type(2)));
+// running maximum of 16 bytes of bf16 magnitudes, two by two: 0x7F80 and above are no numbers
+__device__ __forceinline__ u2_t widest(u2_t top, const uint4& w) {
+  for (const unsigned v : {w.x, w.y, w.z, w.w}) top = __builtin_elementwise_max(top, __builtin_bit_cast(u2_t, v & 0x7FFF7FFFu));
+  return top;
+}
 // row of accumulator entry i (plus 4 in the upper half of the wave)
 __device__ __forceinline__ constexpr int arow(int i) { return 8 * (i / 4) + i % 4; }
 
@@ -77,6 +84,7 @@ __global__ void __launch_bounds__(256, 2) ssd_chunk_kernel(const ScanArgs p) {
   __shared__ __attribute__((aligned(16))) bf16_t sB[kTok * NP];
   __shared__ __attribute__((aligned(16))) bf16_t sC[OUT ? kTok * NP : 8];
   __shared__ __attribute__((aligned(16))) bf16_t sX[kTok * XP];
+  __shared__ int bad[128];  // per column: the first token so far whose x is no number
   __shared__ __attribute__((aligned(16))) float tok[4][5][kTok];  // per wave: c's multiple and rest, dt, end weight, exp(c)
   const int mode = p.mode, np = p.npieces, P = p.dv, H = p.H;
   const int s = blockIdx.z / np, pc = blockIdx.z - s * np;
@@ -134,6 +142,7 @@ __global__ void __launch_bounds__(256, 2) ssd_chunk_kernel(const ScanArgs p) {
     }
     rdt = t0 + lane < qlen ? bf2f(dtp[(row0 + t0 + lane) * p.beta_stride]) : 0.f;
   };
+  if (tid < 128) bad[tid] = std::numeric_limits<int>::max();
   float* my = &tok[wid][0][0];
   double total = 0.0;  // decay exponents of the walk, times log2 e
   fetch(0);
@@ -145,10 +154,24 @@ __global__ void __launch_bounds__(256, 2) ssd_chunk_kernel(const ScanArgs p) {
       *reinterpret_cast<uint4*>(sB + at) = rB[i];
       if constexpr (OUT) *reinterpret_cast<uint4*>(sC + at) = rC[i];
     }
+    u2_t top = {0, 0};
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
       const int id = tid + 256 * i;
       *reinterpret_cast<uint4*>(sX + id / 16 * XP + 8 * (id % 16)) = rX[i];
+      top = widest(top, rX[i]);
+    }
+    // A weight of zero, which later tokens' x have in a token's sum, makes NaN of an x that is no number.  It goes in as zero,
+    // and what its column gives from there on, the state at the end among it, is NaN, as it is token by token.
+    if (max(top[0], top[1]) >= 0x7F80) {
+#pragma unroll 1
+      for (int k = 0; k < 8 * NX; ++k) {
+        const int id = tid + 256 * (k / 8), t = id / 16, at = 8 * (id % 16) + k % 8;
+        if ((sX[t * XP + at] & 0x7F80) == 0x7F80) {
+          sX[t * XP + at] = 0;
+          atomicMin(bad + at, t0 + t);
+        }
+      }
     }
     float eL;
     {  // lane = token
@@ -248,7 +271,14 @@ __global__ void __launch_bounds__(256, 2) ssd_chunk_kernel(const ScanArgs p) {
       }
       __builtin_amdgcn_sched_barrier(0);
       float* op = p.out + static_cast<long>(row0 + t0 + 4 * hi) * (H * P) + hd * P + pcol;
-      const int left = qlen - t0 - 4 * hi;
+      const int left = qlen - t0 - 4 * hi, lost = bad[col0 + c] - t0 - 4 * hi;
+      if (__builtin_amdgcn_ballot_w64(lost < kTok) != 0) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if (32 * t + arow(i) >= lost) acc[t][i] = NAN;
+      }
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -282,12 +312,13 @@ __global__ void __launch_bounds__(256, 2) ssd_chunk_kernel(const ScanArgs p) {
   if (mode == 1 && col0 % P == 0 && lane == 0)  // carries a state across the piece
     p.sc_decay[(static_cast<long>(s) * np + pc) * H + hd] = static_cast<float>(-total * 0.6931471805599453);
   if (mode != 2 || te == qlen_all) {
+    const bool lost = bad[col0 + c] < qlen;
     float* o = (mode == 1 ? p.sc_local + sc_at : slot) + mine;
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
       for (int i = 0; i < 16; i += 4)
-        *reinterpret_cast<f4_t*>(o + 32 * n + arow(i)) = f4_t{S[n][i], S[n][i + 1], S[n][i + 2], S[n][i + 3]};
+        *reinterpret_cast<f4_t*>(o + 32 * n + arow(i)) = lost ? f4_t{NAN, NAN, NAN, NAN} : f4_t{S[n][i], S[n][i + 1], S[n][i + 2], S[n][i + 3]};
   }
 }
 

@@ -64,3 +64,40 @@ def test_decays(gpu, a_mean):
     y, want, st, wst, *_ = run(gpu, 4, 2, 128, 64, [9, 0], [200, 150], a_mean)
     torch.testing.assert_close(y, want, rtol=1e-5, atol=2e-4)
     torch.testing.assert_close(st, wst, rtol=1e-5, atol=2e-4)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("P,N,new", [(64, 128, [100]), (32, 64, [64, 70]), (128, 128, [700])])
+def test_a_token_reaches_no_earlier_one(gpu, P, N, new, bad):
+    """A token whose x, B, C or dt is no number: the outputs before it are what they are without it, its own and later ones are
+    not numbers either (x: in its column alone)."""
+    G, H = 1, max(2, 128 // P)
+    g = torch.Generator().manual_seed(P)
+    T, S = sum(new), len(new)
+    ops = [torch.randn(T, n, generator=g).mul(m).bfloat16() for n, m in ((H * P, 1), (G * N, 0.3), (G * N, 0.3), (H, 1))]
+    dev = [t.to(gpu) for t in (torch.randn(H, generator=g) - 1.0, torch.randn(H, generator=g) - 1.5, torch.randn(H, generator=g))]
+    qsl = torch.tensor([0] + new).cumsum(0).int()
+    lens = torch.tensor(new, dtype=torch.int32)
+
+    def run(ops):
+        pool = torch.zeros(S, H * P * N, device=gpu)
+        y = seqmix.ssd_scan(*(t.to(gpu) for t in ops), *dev, pool, torch.arange(S, dtype=torch.int32, device=gpu), 0, qsl.to(gpu),
+                            lens.to(gpu), H, G, N, P, max(new))
+        return y.cpu(), pool.cpu().view(S, H * P, N)
+
+    clean, st0 = run(ops)
+    a = int(qsl[S - 1])  # the last sequence's
+    for at in (a + 5, a + 31, a + 40, a + 63):
+        for which in range(4):
+            broken = [t.clone() for t in ops]
+            col = P + 3 if which == 0 else 1
+            broken[which][at, col] = bad
+            y, st = run(broken)
+            assert torch.equal(y[:at], clean[:at]), (which, at)
+            if which == 0:
+                others = torch.arange(H * P) != col
+                assert torch.equal(y[:, others], clean[:, others]) and torch.equal(st[:, others], st0[:, others])
+                assert not torch.isfinite(y[at:, col]).any() and not torch.isfinite(st[S - 1, col]).any()
+            elif which == 2:  # C reads the state and leaves none of it behind
+                assert not torch.isfinite(y[at]).any() and torch.equal(st, st0)
+                assert torch.equal(y[at + 1:], clean[at + 1:])
