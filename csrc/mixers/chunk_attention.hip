@@ -287,6 +287,72 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
     }
     if (it + 1 < itn) put_tile(lds[(it + 1) & 1]);
   }
+  // A weight of zero makes NaN of a value that is no number, in queries that do not see its key: entries that came out as no
+  // numbers are summed again key by key over the keys that their query does see, until no number can come of them any more.
+  float odd = 0.f;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) odd = fmaf(o[dt][i], 0.f, odd);
+  if (__builtin_amdgcn_ballot_w64(odd != 0.f) != 0) {
+    f16_t r[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) r[dt][i] = 0.f;
+    bool open = true;
+#pragma unroll 1
+    for (int n = it0 * KT; n < itn * KT && open; ++n) {
+      const int j = start_of(n / KT) + n % KT;
+      if (j < low0 || j > min(kmax, whi)) continue;
+      const bf16_t *kj, *vj, *rj = nullptr;
+      if constexpr (PAGED) {
+        const bf16_t* blk = a.cache + static_cast<long>(bt[min(j >> 4, lastpage)]) * a.block_stride;
+        kj = blk + a.koff + (g * 16 + (j & 15)) * dk;
+        vj = blk + a.voff + (g * 16 + (j & 15)) * dv;
+      } else {
+        const long row = dense0 + j;
+        kj = a.kx + row * a.x_stride + g * a.dn;
+        vj = a.vx + row * a.x_stride + g * dv;
+        rj = a.kr + row * a.r_stride - a.dn;
+      }
+      float sc = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int d = 16 * ks + 8 * hi;
+        if (d >= dk) continue;
+        float x[8];
+        load16((PAGED || d < a.dn ? kj : rj) + d, x);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sc = fmaf(static_cast<float>(qf[ks][e]), x[e], sc);
+      }
+      sc = across(sc, true);
+      const bool seen = (j <= pos) & ((j > low) | (j < a.keep));
+      const float w = __builtin_amdgcn_exp2f(fmaf(sc, sl2, m == -INFINITY ? 0.f : -m));
+      open = false;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const int d = 32 * dt + 8 * b + 4 * hi;
+          if (d >= dv) continue;
+          const uint2 v = *reinterpret_cast<const uint2*>(vj + d);
+          const float x[4] = {bf2f_lo(v.x), bf2f_hi(v.x), bf2f_lo(v.y), bf2f_hi(v.y)};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int i = 4 * b + e;
+            if (seen) r[dt][i] = fmaf(w, x[e], r[dt][i]);
+            open |= !(fabsf(o[dt][i]) < INFINITY) && fabsf(r[dt][i]) < INFINITY;
+          }
+        }
+      open = __builtin_amdgcn_ballot_w64(open) != 0;
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (!(fabsf(o[dt][i]) < INFINITY)) o[dt][i] = r[dt][i];
+  }
   l = across(l, true);
   if (!qok) return;
   if constexpr (SPLIT) {

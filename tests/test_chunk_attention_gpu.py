@@ -89,3 +89,41 @@ def test_other_strides_and_scales(gpu):
     check(gpu, 4, 2, 64, 64, [(0, 40), (70, 50)], scale=-0.2, pad=4, sink=True)  # rows on 8-byte borders, a negative scale
     check(gpu, 2, 2, 64, 64, [(0, 40)], scale=0.0)
     check(gpu, 2, 1, 128, 64, [(9, 40)], scale=3.0, pad=12)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("H,G,dk,dv", [(4, 4, 64, 64), (8, 2, 64, 48), (2, 2, 128, 96), (4, 1, 96, 128)])
+@pytest.mark.parametrize("past,new,window,keep", [(0, 140, 0, 0), (70, 200, 90, 5), (2100, 40, 0, 0)])
+def test_a_token_reaches_only_queries_that_see_it(gpu, H, G, dk, dv, past, new, window, keep, bad):
+    """A token with a value (or a key) that is no number: queries that do not see it give what they give without it, those that
+    do are no numbers in that entry (a key: in all of them)."""
+    g = torch.Generator().manual_seed(dk + new)
+    n = past + new
+    nb = -(-n // PAGE)
+    koff, voff = 0, G * PAGE * dk
+    cache = torch.randn(nb, voff + G * PAGE * dv, generator=g).bfloat16()
+    q = torch.randn(new, H * dk, generator=g).bfloat16()
+    bt = torch.arange(nb, dtype=torch.int32).view(1, nb)
+
+    def run(c):
+        return seqmix.window_attention(q.to(gpu), c.to(gpu), bt.to(gpu), torch.tensor([0, new], dtype=torch.int32, device=gpu),
+                                       torch.tensor([n], dtype=torch.int32, device=gpu), koff, voff, H, G, dk, dv, PAGE, dk ** -0.5,
+                                       window, keep, new, max_seq_len=n).cpu().float().view(new, H, dv)
+
+    clean = run(cache)
+    i = torch.arange(past, n)
+    group = torch.arange(H) // (H // G) == G - 1
+    for j in sorted({3, past + 1, past + 17, past + 31, past + 39, n - 30, n - 2}):
+        seen = (i >= j) & ((i - j < window) | (j < keep) if window > 0 else torch.tensor(True))
+        for off, d, col in ((voff, dv, dv - 1), (koff, dk, 2)):
+            c = cache.clone()
+            c[j // PAGE, off + ((G - 1) * PAGE + j % PAGE) * d + col] = bad
+            y = run(c)
+            hit = torch.zeros(new, H, dv, dtype=torch.bool)
+            cols = torch.arange(dv) == col if off == voff else torch.ones(dv, dtype=torch.bool)
+            hit |= seen[:, None, None] & group[None, :, None] & cols[None, None, :]
+            # another tile's maximum may set the reference that weights are scaled by: fp32 roundings, one of bf16 at the end
+            err = ((y - clean).abs() - 2.0 ** -7 * clean.abs())[~hit]
+            assert not err.numel() or float(err.max()) <= 2.0 ** -12, (j, off == voff, float(err.max()))
+            if bad != bad:
+                assert not torch.isfinite(y[hit]).any(), (j, off == voff)

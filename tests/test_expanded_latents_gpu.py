@@ -164,3 +164,24 @@ def test_mixer_expands_and_folds(gpu, monkeypatch, window, singles):
     err = {k: float((o - want).norm() / want.norm()) for k, o in outs.items()}
     # the chain of bf16 roundings (projections, rows, keys, values, outputs): about six of 2^-9 each
     assert err["folded"] < 0.012 and err["expanded"] < 0.012 and err["expanded"] < 1.2 * err["folded"], err
+
+
+@pytest.mark.parametrize("past,new,window", [(0, 140, 0), (75, 130, 50)])
+def test_a_value_reaches_only_queries_that_see_it(gpu, past, new, window):
+    """A gathered row whose expanded value is no number: queries that do not see its key give what they give without it."""
+    H, dn, dr, dv, rank = 2, 64, 32, 96, 64
+    g = torch.Generator().manual_seed(past)
+    qsl, lens = torch.tensor([0, new], dtype=torch.int32, device=gpu), torch.tensor([past + new], dtype=torch.int32, device=gpu)
+    base, offs = seqmix.latent_plan(qsl, lens, window)
+    n, b = int(offs[1]), int(base[0])
+    q, kv, rows = (torch.randn(*s, generator=g).bfloat16().to(gpu) for s in ((new, H * (dn + dr)), (n, H * (dn + dv)), (n, rank + dr)))
+    run = lambda kv: seqmix.expanded_attention(q, kv, rows, base, qsl, lens, H, dn, dr, dv, 0.1, new, None, window).cpu().float()  # noqa: E731
+    clean, i = run(kv), past + torch.arange(new)
+    for j in (past + 3, past + 40, past + 63, past + new - 2, max(past - 20, 0)):
+        broken = kv.clone()
+        broken[b + j, H * dn + dv + 5] = float("nan")  # head 1, entry 5
+        y = run(broken).view(new, H, dv)
+        seen = (i >= j) & ((i - j < window) if window > 0 else torch.tensor(True))
+        assert not torch.isfinite(y[seen, 1, 5]).any()
+        y[seen, 1, 5] = clean.view(new, H, dv)[seen, 1, 5]
+        torch.testing.assert_close(y.view(new, -1), clean, rtol=2.0 ** -7, atol=2.0 ** -12)
