@@ -14,8 +14,9 @@
 //   accumulators hold it), the parts meet in LDS over one barrier a chunk.
 // Bound by the walk's chain (48 matrix instructions of 32 cycles, a turn through LDS, and one wave a SIMD to hide them).  4,096
 // tokens, 16 heads of 128 x 128: 1,480 us token by token (in pieces of 256, each carrying its transition matrix of 128 more
-// columns, twice, with library products in between), 437 us here, 154 of them the preparation.  Error against 64 bits, of the
-// outputs' norm: half lives of a thousand tokens 9.7e-7 before, 2.7e-7 here; of some tokens 1.34e-7 and 1.31e-7.
+// columns, twice, with library products in between), 432 us here, 156 of them the preparation.  Error against 64 bits, of a
+// head's outputs / its state after 96 tokens, by tokens -> here: half lives of a thousand tokens 3.6e-7 -> 1.8e-7 / 4.5e-7 ->
+// 2.0e-7, of some tokens 1.36e-7 -> 1.25e-7 / 1.07e-7 -> 1.02e-7, of a tenth of a token 1.21e-7 -> 1.13e-7 / 8.5e-8 -> 7.9e-8.
 #include <algorithm>
 
 #include "mix_common.h"
@@ -37,6 +38,10 @@ __device__ __forceinline__ float row16(float v) {  // sum over 16 lanes of a DPP
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, false));
   return v;
 }
+// What scales a whole row is not rounded before it does, or once: a chunk's sums round a little more often than a walk by tokens,
+// and where decays are fast, so that nothing else is left, that was 2 to 7 % of the error.
+__device__ __forceinline__ double unit_of(float square, float scale) { return static_cast<double>(scale) / sqrt(static_cast<double>(square)); }
+__device__ __forceinline__ float strength(float z) { return static_cast<float>(1.0 / (1.0 + exp(-static_cast<double>(z)))); }
 // a barrier for LDS alone: __syncthreads would wait for the loads of the chunks to come as well
 __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -105,17 +110,17 @@ __global__ void __launch_bounds__(256) delta_prepare_kernel(const ScanArgs p, fl
       sq += q[i] * q[i];
     }
     const bool in = t < nt;
-    const float ik = rsqrtf(row16(sk) + p.unit_eps), iq = rsqrtf(row16(sq) + p.unit_eps) * p.q_scale;
+    const double ik = unit_of(row16(sk) + p.unit_eps, 1.f), iq = unit_of(row16(sq) + p.unit_eps, p.q_scale);
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       const int d = part * R + i;
-      ks[t][d] = in ? k[i] * ik : 0.f;
-      qs[t][d] = in ? q[i] * iq : 0.f;
+      ks[t][d] = in ? static_cast<float>(k[i] * ik) : 0.f;
+      qs[t][d] = in ? static_cast<float>(q[i] * iq) : 0.f;
       const float l = in ? eA * softplus_d(a[i] + p.dt_bias[hd * DK + d]) : 0.f;
       ls[t][d] = l;
       gs[t][d] = expf(-l);
     }
-    if (part == 0) bs[t] = in ? sigmoid_f(bf2f(static_cast<const bf16_t*>(p.beta)[row * p.beta_stride + hd])) : 0.f;
+    if (part == 0) bs[t] = in ? strength(bf2f(static_cast<const bf16_t*>(p.beta)[row * p.beta_stride + hd])) : 0.f;
   }
   __syncthreads();
   {  // A and Q of keys grp and grp + 16

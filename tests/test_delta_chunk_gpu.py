@@ -69,3 +69,30 @@ def test_decays(gpu, a_mean):
     y, want, st, wst, *_ = run(gpu, 2, 1, 128, 64, [9, 0], [200, 150], a_mean)
     torch.testing.assert_close(y, want, rtol=1e-5, atol=1e-4)
     torch.testing.assert_close(st, wst, rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("a_mean", [-8.0, -2.0, 0.0, 1.0, 2.0, 4.0, 6.0])
+def test_no_further_off_than_token_by_token(gpu, monkeypatch, a_mean, dim):
+    """From half lives of a thousand tokens to resets by each: the chunks' error against 64 bits, as a share of the norm of a head's
+    outputs and state and on average over a thousand heads, is no larger than that of the walk by tokens."""
+    H, T = 64, 80
+    err = {0: [], 1 << 40: []}
+    for seed in range(16):
+        g = torch.Generator(device=gpu).manual_seed(seed)
+        rnd = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
+        q, k, v, b, a = (rnd(T, n).bfloat16() for n in (H * dim, H * dim, H * dim, H, H * dim))
+        dtb, A = rnd(H * dim) - 1.0, rnd(H) * 0.5 + a_mean
+        st = torch.zeros(1, H, dim, dim, dtype=torch.float64, device=gpu)
+        with torch.device(gpu):
+            want = reference(*(t.double() for t in (q, k, v, b, a, dtb, A)), st, [0], [T], H, H, dim, dim, dim ** -0.5)
+        for least, e in err.items():
+            monkeypatch.setattr(seqmix, "DELTA_CHUNK_TOKENS", least)
+            pool = torch.zeros(1, H * dim * dim, device=gpu)
+            ints = [torch.tensor(x, dtype=torch.int32, device=gpu) for x in ([0], [0, T], [T])]
+            y = seqmix.delta_scan(q, k, v, b, a, dtb, A, pool, ints[0], 0, ints[1], ints[2], H, H, dim, dim, dim ** -0.5, max_query_len=T)
+            share = lambda x, w, d: (x - w).norm(dim=d) / w.norm(dim=d)  # noqa: E731
+            e.append(torch.stack([share(y.double().view(T, H, dim), want.view(T, H, dim), (0, 2)),
+                                  share(pool.double().view(H, -1), st.view(H, -1), 1)], 1))
+    chunks, tokens = (torch.cat(e).mean(0).tolist() for e in err.values())
+    assert chunks[0] <= tokens[0] and chunks[1] <= tokens[1], (chunks, tokens)
