@@ -11,8 +11,9 @@
 // heads of a B/C group, which share the 64 rows of B, C and x in LDS.  The next tile's pieces are in flight in registers under
 // the products of the state.  Long chunks are cut into pieces as in column_scan.hip (its modes and its chain).
 // Bound by instruction issue (138 matrix instructions a chunk and wave beside some 2,000 others): 4,096 tokens, 64 heads of
-// 64, state 128, both passes: 720 us token by token on the vector units, 125 us
-// here, and with less error against 64 bits (2e-7 of y's norm against 5e-7 at half lives of a thousand tokens).
+// 64, state 128, both passes: 720 us token by token on the vector units, 114 us here.  Error against 64 bits, of a head's outputs /
+// its state after 96 tokens, by tokens -> here: half lives of thousands of tokens 3.1e-7 -> 1.25e-7 / 4.3e-7 -> 1.1e-7, of some
+// tokens 7.9e-8 -> 7.0e-8 / 8.1e-8 -> 5.9e-8, of a fraction of one 6.6e-8 -> 6.4e-8 / 7.9e-8 -> 5.8e-8.
 #include <algorithm>
 #include <limits>
 
@@ -70,6 +71,25 @@ typedef unsigned short u2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ u2_t widest(u2_t top, const uint4& w) {
   for (const unsigned v : {w.x, w.y, w.z, w.w}) top = __builtin_elementwise_max(top, __builtin_bit_cast(u2_t, v & 0x7FFF7FFFu));
   return top;
+}
+// softplus(a + b) = max(z, 0) + log(1 + exp(-|z|)) to one rounding: every step keeps what it rounds away.  Everything that a
+// token writes and shows goes through this number, so that its error, unlike a sum's, does not average out.  The exponential
+// by its series after a whole power of two is taken out, the logarithm as 2 atanh(e / (2 + e)) by its series.
+__device__ __forceinline__ float softplus_sum(float a, float b) {
+  const float z = a + b, zb = z - a, u = fminf(fabsf(z), 200.f);
+  const float zl = u < 200.f ? (a - (z - zb)) + (b - zb) : 0.f, n = rintf(u * -1.44269504f);
+  const float r0 = fmaf(n, -0.693145752f, -u);                    // 16 bits of ln 2: exact
+  const float r1 = fmaf(n, -1.42860677e-6f, z > 0.f ? -zl : zl);  // and the rest of it
+  const float r = r0 + r1, rl = (r0 - r) + r1;
+  const float p = r * r * fmaf(r, fmaf(r, fmaf(r, fmaf(r, fmaf(r, fmaf(r, 1.f / 40320, 1.f / 5040), 1.f / 720), 1.f / 120), 1.f / 24), 1.f / 6), 0.5f);
+  const float q = p + rl, s = r + q, sl = (r - s) + q, eh = 1.f + s;
+  const float e = ldexpf(eh, static_cast<int>(n)), el = ldexpf(((1.f - eh) + s) + sl, static_cast<int>(n));
+  const float t = 2.f + e, tl = (e - (t - 2.f)) + el, rc = __builtin_amdgcn_rcpf(t);
+  const float h = e * rc, hl = (fmaf(-h, t, e) + fmaf(-h, tl, el)) * rc, h2 = h * h;
+  const float k = h2 * fmaf(h2, fmaf(h2, fmaf(h2, fmaf(h2, fmaf(h2, fmaf(h2, fmaf(h2, 1.f / 17, 1.f / 15), 1.f / 13), 1.f / 11), 1.f / 9), 1.f / 7), 1.f / 5), 1.f / 3);
+  const float L = 2.f * h, Ll = 2.f * fmaf(h, k, fmaf(hl, h2, hl));
+  const float m = z < 0.f ? 0.f : z, y = m + L, yb = y - m;
+  return m < 1e30f ? y + ((m - (y - yb)) + (L - yb) + (Ll + (z > 0.f ? zl : 0.f))) : m;
 }
 // row of accumulator entry i (plus 4 in the upper half of the wave)
 __device__ __forceinline__ constexpr int arow(int i) { return 8 * (i / 4) + i % 4; }
@@ -176,8 +196,8 @@ __global__ void __launch_bounds__(256, 2) ssd_chunk_kernel(const ScanArgs p) {
     float eL;
     {  // lane = token
       const bool in = t0 + lane < qlen;
-      const float z = rdt + bias, dt = in ? fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))) : 0.f;
-      double cum = in ? -static_cast<double>(fminf(eA * dt, 128.f)) * 1.4426950408889634 : 0.0;
+      const float dt = in ? softplus_sum(rdt, bias) : 0.f;
+      double cum = in ? -fmin(static_cast<double>(eA) * dt, 128.0) * 1.4426950408889634 : 0.0;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
         const double up = __shfl_up(cum, o, 64);
@@ -236,14 +256,17 @@ __global__ void __launch_bounds__(256, 2) ssd_chunk_kernel(const ScanArgs p) {
 #pragma unroll
         for (int u = 0; u <= t; ++u) {
           __builtin_amdgcn_sched_barrier(0);
-          f16_t g;
+          f16_t g, g2;  // two sums where the registers hold them: half as many roundings at the size of the whole
+          constexpr bool kTwo = NT == 2;
 #pragma unroll
-          for (int i = 0; i < 16; ++i) g[i] = 0.f;
+          for (int i = 0; i < 16; ++i) g[i] = g2[i] = 0.f;
 #pragma unroll
           for (int j = 0; j < 2 * NT; ++j) {
             if (j % 2 == 0) __builtin_amdgcn_sched_barrier(0);
-            g = mm(row_perm(sB + (32 * u + c) * NP + 16 * j + 4 * hi), row_perm(sC + (32 * t + c) * NP + 16 * j + 4 * hi), g);
+            f16_t& sum = kTwo && j % 2 ? g2 : g;
+            sum = mm(row_perm(sB + (32 * u + c) * NP + 16 * j + 4 * hi), row_perm(sC + (32 * t + c) * NP + 16 * j + 4 * hi), sum);
           }
+          if constexpr (kTwo) g += g2;
 #pragma unroll
           for (int i = 0; i < 16; i += 4) {
             __builtin_amdgcn_sched_barrier(0);

@@ -101,3 +101,56 @@ def test_a_token_reaches_no_earlier_one(gpu, P, N, new, bad):
             elif which == 2:  # C reads the state and leaves none of it behind
                 assert not torch.isfinite(y[at]).any() and torch.equal(st, st0)
                 assert torch.equal(y[at + 1:], clean[at + 1:])
+
+
+@pytest.mark.parametrize("H,G,N,P", [(64, 8, 128, 64), (64, 4, 64, 128)])
+@pytest.mark.parametrize("a_mean", [-8.0, -2.0, 0.0, 1.0, 2.0, 3.0, 7.0])
+def test_no_further_off_than_token_by_token(gpu, a_mean, H, G, N, P):
+    """From half lives of thousands of tokens to a reset by each: the error against 64 bits, as a share of the norm of a head's
+    outputs and state and on average over a thousand heads, is no larger than that of the walk by tokens."""
+    T = 80
+    err = {"chunks": [], "tokens": []}
+    for seed in range(16):
+        g = torch.Generator(device=gpu).manual_seed(seed)
+        rnd = lambda *s: torch.randn(*s, generator=g, device=gpu)  # noqa: E731
+        x, B, C, dt = (rnd(T, n).mul(m).bfloat16() for n, m in ((H * P, 1), (G * N, 0.3), (G * N, 0.3), (H, 1)))
+        dtb, A, D = rnd(H) - 1.0, rnd(H) * 0.5 + a_mean, rnd(H)
+        st = torch.zeros(1, H, P, N, dtype=torch.float64, device=gpu)
+        shaped = (t.double().view(T, *s) for t, s in ((x, (H, P)), (B, (G, N)), (C, (G, N)), (dt, (H,))))
+        want = reference(*shaped, dtb.double(), A.double(), D.double(), st, [0], [T], G)
+        odd = torch.zeros(T, H * P + 1, dtype=x.dtype, device=gpu)
+        odd[:, 1:] = x  # no whole 16-byte pieces: token by token
+        for way, xs in (("chunks", x), ("tokens", odd[:, 1:])):
+            pool = torch.zeros(1, H * P * N, device=gpu)
+            ints = [torch.tensor(v, dtype=torch.int32, device=gpu) for v in ([0], [0, T], [T])]
+            y = seqmix.ssd_scan(xs, B, C, dt, dtb, A, D, pool, ints[0], 0, ints[1], ints[2], H, G, N, P, T)
+            share = lambda v, w, d: (v - w).norm(dim=d) / w.norm(dim=d)  # noqa: E731
+            err[way].append(torch.stack([share(y.double().view(T, H, P), want, (0, 2)),
+                                         share(pool.double().view(H, -1), st.view(H, -1), 1)], 1))
+    chunks, tokens = (torch.cat(e).mean(0).tolist() for e in err.values())
+    assert chunks[0] <= tokens[0] and chunks[1] <= tokens[1], (chunks, tokens)
+
+
+def test_softplus_of_a_sum(gpu):
+    """The step sizes over the whole range, shown by a state that starts empty and one token: S = dt x B."""
+    H, N, P, T = 2, 64, 64, 64
+    worst = 0.0
+    for bias in (-30.0, -9.5, -1.0, -1e-3, 0.0, 0.7, 3.3, 25.0):
+        dt = torch.linspace(-60, 60, 4001).bfloat16()
+        for v in dt[:: 211].tolist():
+            x, B = torch.ones(T, H * P).bfloat16(), torch.zeros(T, N).bfloat16()
+            B[0, 0] = 1.0
+            x[1:] = 0.0
+            d = torch.full((T, H), -1e30).bfloat16()
+            d[0] = v
+            pool = torch.zeros(1, H * P * N, device=gpu)
+            ints = [torch.tensor(i, dtype=torch.int32, device=gpu) for i in ([0], [0, T], [T])]
+            b = torch.full((H,), bias)
+            seqmix.ssd_scan(x.to(gpu), B.to(gpu), B.to(gpu), d.to(gpu), b.to(gpu), torch.zeros(H, device=gpu), torch.zeros(H, device=gpu),
+                            pool, ints[0], 0, ints[1], ints[2], H, 1, N, P, T)
+            z = torch.tensor(v, dtype=torch.float64) + float(b[0])
+            want = float(torch.clamp(z, min=0) + torch.log1p(torch.exp(-z.abs())))
+            got = float(pool[0, 0])
+            if want > 1e-36:
+                worst = max(worst, abs(got - want) / want)
+    assert worst <= 2.0 ** -23, worst  # one rounding (2^-24), and as much for what the steps before it keep of theirs
