@@ -6,6 +6,8 @@
 //                              graph-capturable, no RNG state).  No sort: the top-k and top-p
 //                              thresholds come from a histogram of the row (select_threshold).
 // The hash matches mxserve/ops/reference.py::_hash_u32 bit for bit.
+#include <cstdlib>
+
 #include "common.h"
 
 namespace mxs {
@@ -346,17 +348,22 @@ void launch_sample(int64_t* out, const void* logits, bool bf16, int B, int V, lo
   auto run = [&](auto kernel, auto* z) {
     hipLaunchKernelGGL(kernel, dim3(B), dim3(1024), 0, s, out, z, V, row_stride, vec, temperature, top_p, top_k, seeds, steps);
   };
+  static const bool reg_ok = [] {  // MXS_SAMPLE_REG=0: rows are read again by each pass (the same tokens)
+    const char* e = std::getenv("MXS_SAMPLE_REG");
+    return e == nullptr || e[0] != '0';
+  }();
   // registers hold a row up to what 1024 threads of 128 VGPRs have room for: 160 bf16 or 64 fp32 logits a thread
+  const int fit = vec && reg_ok ? V : 1 << 30;
   if (bf16) {
     const auto* z = static_cast<const bf16_t*>(logits);
-    if (vec && V <= 1024 * 32) run(sample_kernel<RegRow16<32>>, z);
-    else if (vec && V <= 1024 * 128) run(sample_kernel<RegRow16<128>>, z);
-    else if (vec && V <= 1024 * 160) run(sample_kernel<RegRow16<160>>, z);
+    if (fit <= 1024 * 32) run(sample_kernel<RegRow16<32>>, z);
+    else if (fit <= 1024 * 128) run(sample_kernel<RegRow16<128>>, z);
+    else if (fit <= 1024 * 160) run(sample_kernel<RegRow16<160>>, z);
     else run(sample_kernel<MemRow<bf16_t>>, z);
   } else {
     const auto* z = static_cast<const float*>(logits);
-    if (vec && V <= 1024 * 32) run(sample_kernel<RegRow32<32>>, z);
-    else if (vec && V <= 1024 * 64) run(sample_kernel<RegRow32<64>>, z);
+    if (fit <= 1024 * 32) run(sample_kernel<RegRow32<32>>, z);
+    else if (fit <= 1024 * 64) run(sample_kernel<RegRow32<64>>, z);
     else run(sample_kernel<MemRow<float>>, z);
   }
   MXS_CHECK_LAUNCH();
