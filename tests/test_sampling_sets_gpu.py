@@ -94,3 +94,24 @@ def test_many_small_shares_count(gpu, dtype, V):
     got = ops.sample(z.view(1, V).to(gpu), one(1.0, torch.float32), one(p, torch.float32), one(0, torch.int32),
                      one(seed, torch.int64), one(2, torch.int64))
     assert int(got[0]) == mid
+
+
+@pytest.mark.parametrize("V", [5, 8, 1000, 8192, 8200, 24576, 32768, 32776, 65544, 163848])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_of_one_pass(gpu, dtype, V):
+    """Greedy rows and draws without a set, which no register form holds: every place of a row can win, the last one too."""
+    g = torch.Generator().manual_seed(V)
+    best = sorted({0, V // 2, V - 1, V * 3 // 4, min(V - 1, 8191), min(V - 1, 16384)})
+    B = 2 * len(best)
+    z = (torch.randn(B, V, generator=g) * 0.5).clamp(-2, 2).to(dtype)
+    temp = torch.tensor([0.0, 0.8] * len(best))
+    seeds, steps = torch.arange(B), torch.full((B,), 3)
+    for i, v in enumerate(best):
+        z[2 * i, v] = 3.0
+    got = ops.sample(z.to(gpu), temp.to(gpu), torch.ones(B, device=gpu), torch.zeros(B, dtype=torch.int32, device=gpu),
+                     seeds.to(gpu), steps.to(gpu)).cpu()
+    assert got[::2].tolist() == best
+    noise = -torch.log(-torch.log(ref.uniform_noise(seeds[1::2], steps[1::2], V).double()))
+    score = z[1::2].double() / 0.8 + noise
+    # the kernel's noise is two fp32 logarithms: 2^-20 of a score of at most 20
+    assert (score.max(-1).values - score.gather(1, got[1::2, None])[:, 0] <= 2e-5).all()
