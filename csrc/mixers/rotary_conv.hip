@@ -294,8 +294,9 @@ __global__ void __launch_bounds__(256) causal_conv_kernel(T* __restrict__ out, c
 
 // The wide form for chunks: a thread takes its channels of 4 consecutive rows, so that a row is read once and not once per
 // tap; what a row's filter reaches back to is carried from row to row, and taken anew where a sequence begins.  The terms
-// of a sum are those of the kernel above, in its order.  4,096 rows of 6,144 channels, 4 taps: 48 -> 37 us.
+// of a sum are those of the kernel above, in its order.  4,096 rows of 6,144 channels, 4 taps: 46 -> 34 us.
 constexpr int kConvRows = 4;
+constexpr long kConvBytes = 7 << 20;
 template <typename T, int TAPS>
 __global__ void __launch_bounds__(256) causal_conv_rows_kernel(T* __restrict__ out, const T* __restrict__ x, long x_stride,
                                                                const T* __restrict__ w, const T* __restrict__ bias,
@@ -633,14 +634,18 @@ void launch_causal_conv(void* out, const void* x, long x_stride, const void* w, 
   auto al = [](const void* ptr) { return reinterpret_cast<uintptr_t>(ptr) % 16 == 0; };
   const bool wide = C % v == 0 && x_stride % v == 0 && al(x) && al(w) && al(out) && (bias == nullptr || al(bias)) &&
                     al(state) && state_stride % 4 == 0 && off % 4 == 0;
-  if (wide && !single && taps >= 2 && taps <= 4) {
+  // Four rows a thread where the bytes count: below some 7 MB of rows a quarter of the workgroups and a chain of four rows take
+  // longer than reading rows again, most of all for few channels (bf16, 4 taps, one row a thread / four: 4,096 rows of 64
+  // 7.9 / 16.0 us, 2,048 of 1,024 8.0 / 10.1, 1,024 of 3,072 10.3 / 10.6, 700 of 5,120 12.3 / 12.2, 2,048 of 2,048 13.1 / 11.1,
+  // 4,096 of 6,144 46.1 / 34.4; fp32, 2,048 of 512 6.6 / 7.3, 512 of 3,072 8.5 / 7.8).  Two taps read too little twice: 4,096 of
+  // 3,072 20.4 / 21.3.
+  if (wide && !single && (taps == 3 || taps == 4) && static_cast<long>(rows) * C * (16 / v) >= kConvBytes) {
     const dim3 grid((rows + kConvRows - 1) / kConvRows, (C / v + 255) / 256);
 #define MIX_CONV(TAPS)                                                                                                    \
   MIX_DISPATCH(bf, hipLaunchKernelGGL((causal_conv_rows_kernel<T, TAPS>), grid, dim3(256), 0, st, (T*)out, (const T*)x,   \
                                       x_stride, (const T*)w, (const T*)bias, state, state_stride, state_rows, off, qsl,  \
                                       seq_lens, S, rows, C, silu))
-    if (taps == 2) MIX_CONV(2);
-    else if (taps == 3) MIX_CONV(3);
+    if (taps == 3) MIX_CONV(3);
     else MIX_CONV(4);
 #undef MIX_CONV
   } else if (wide) {

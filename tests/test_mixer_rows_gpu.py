@@ -92,6 +92,35 @@ def test_convolution_rows(gpu, dt, C, taps, lens):
 
 
 @pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("lens", [[3, 4, 1, 2, 17, 9], [1], [2001], [0, 7, 1, 8, 0, 16]])
+@pytest.mark.parametrize("more", [0, 3])
+def test_convolution_of_many_rows(gpu, dt, taps, lens, more):
+    """Enough rows and channels for four rows a thread (and, in the last line, just too few for it): groups of four across
+    borders of sequences, also of empty ones, and rows past the last sequence."""
+    g = torch.Generator().manual_seed(taps + len(lens) + more)
+    for C, least in ((2056, 1840 if dt == torch.bfloat16 else 920), (2056, 1770 if dt == torch.bfloat16 else 880)):
+        n = lens * max(1, -(-least // sum(lens)))
+        T, S = sum(n) + more, len(n)
+        x, b = torch.randn(T, C + 16, generator=g).to(dt)[:, 16:], torch.randn(C, generator=g).to(dt)
+        w = torch.randn(taps, C, generator=g).to(dt)
+        state = torch.randn(S + 2, 8 + (taps - 1) * C, generator=g)
+        rows = torch.randperm(S + 2, generator=g)[:S].int()
+        qsl = torch.tensor([0] + n).cumsum(0).int()
+        seq = torch.tensor([m + (0 if i % 2 else 9) for i, m in enumerate(n)], dtype=torch.int32)
+        sg = state.to(gpu)
+        got = seqmix.causal_conv(x.to(gpu), w.to(gpu), b.to(gpu), sg, rows.to(gpu), 8, qsl.to(gpu), seq.to(gpu), True, max(2, max(n)))
+        sc, end, last = state.clone(), qsl.clone(), S - 1
+        seqmix.causal_conv(x[:T - more], w, b, sc, rows, 8, qsl, seq, True, max(n))
+        torch.testing.assert_close(sg.cpu(), sc, rtol=0, atol=0)
+        if more:  # they go on as the last sequence's
+            end[S] = T
+            seq = seq + torch.tensor([0] * last + [more], dtype=torch.int32)
+        want = seqmix.causal_conv(x, w, b, state.clone(), rows, 8, end, seq, True, T)
+        torch.testing.assert_close(got.cpu().float(), want.float(), **tol(dt))
+
+
+@pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("taps", [2, 4])
 @pytest.mark.parametrize("lens", [[3], [5, 2], [4, 9, 0], [1, 1, 1]])
 @pytest.mark.parametrize("more", [1, 2, 7])
