@@ -144,8 +144,8 @@ __global__ void __launch_bounds__(512) rope_qkv_cache_wide_kernel(
     const T* __restrict__ q_norm, const T* __restrict__ k_norm, float eps, const float* __restrict__ v_freqs, int nvf) {
   extern __shared__ float2 cs[];  // [nf] then [nvf]
   const long t = blockIdx.x;
-  const int LP = dk / 8, nq = H * LP, nk = k ? G * LP : 0, n = nq + nk + (k ? G * dv / 8 : 0);
-  int i = threadIdx.x;
+  const int LP = dk / 8, nq = H * LP, nk = k ? G * LP : 0, n = nq + nk + (k ? G * dv / 8 : 0), step = blockDim.x * gridDim.y;
+  int i = blockIdx.y * blockDim.x + threadIdx.x;
   float x[8];
   auto fetch = [&] {
     if (i < n) ld8f(i < nq ? q + t * q_stride + 8 * i : i < nq + nk ? k + t * k_stride + 8 * (i - nq) : v + t * v_stride + 8 * (i - nq - nk), x);
@@ -158,7 +158,7 @@ __global__ void __launch_bounds__(512) rope_qkv_cache_wide_kernel(
   __syncthreads();
   T* page = cache + (slot < 0 ? 0 : slot / bs) * block_stride;
   const int off = static_cast<int>(slot < 0 ? 0 : slot % bs);
-  for (; i < n; i += blockDim.x, fetch()) {
+  for (; i < n; i += step, fetch()) {
     if (i < nq + nk) {
       const bool isq = i < nq;
       const int j = isq ? i : i - nq, d = 8 * (j % LP), head = j / LP;
@@ -192,8 +192,8 @@ __global__ void __launch_bounds__(256) rope_rows_wide_kernel(T* __restrict__ out
                                                              float scale) {
   extern __shared__ float2 cs[];
   const long t = blockIdx.x;
-  const int n = heads * dim / 8;
-  int i = threadIdx.x;
+  const int n = heads * dim / 8, step = blockDim.x * gridDim.y;
+  int i = blockIdx.y * blockDim.x + threadIdx.x;
   float v[8];
   if (i < n) ld8f(x + t * x_stride + 8 * i, v);
   make_turns(cs, freqs, nf, static_cast<float>(positions[t]) * sign);
@@ -203,7 +203,7 @@ __global__ void __launch_bounds__(256) rope_rows_wide_kernel(T* __restrict__ out
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] *= scale;
     st8f(out + t * out_stride + 8 * i, v);
-    if ((i += blockDim.x) < n) ld8f(x + t * x_stride + 8 * i, v);
+    if ((i += step) < n) ld8f(x + t * x_stride + 8 * i, v);
   }
 }
 
@@ -579,6 +579,12 @@ void launch_embed_scaled(float* out, const int64_t* ids, const void* table, int 
   MXS_CHECK_LAUNCH();
 }
 
+// The form with a wave per token and head is faster while the chip holds all waves at once (7 tokens of 32 + 8 + 8 heads
+// of 64 3.3 us, 4.0 here; 64 tokens 3.7 / 4.1; 200 tokens 5.2 / 4.2) or a token has no more pieces than a wave lanes (64
+// tokens of 4 + 2 + 2 heads of 64 3.3 / 4.4; 4,096 tokens of one head of 8 6.1 / 7.1).  Up to kFewRows tokens, a token's pieces go over as many workgroups as hold them (64 tokens of
+// 128 + 8 + 8 heads of 128: 7.1 us with one, 4.7).
+constexpr int kFewRows = 256, kFewPieces = 64, kFewWaves = 4096;
+
 void launch_rope_qkv_cache(void* q, long q_stride, const void* k, long k_stride, const void* v, long v_stride,
                            const int64_t* positions, const int64_t* slots, void* cache, long block_stride, int rows,
                            int koff, int voff, int H, int G, int dk, int dv, int bs, const float* freqs, int nf,
@@ -586,15 +592,16 @@ void launch_rope_qkv_cache(void* q, long q_stride, const void* k, long k_stride,
                            hipStream_t st) {
   if (rows == 0) return;
   auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  const int LP = dk / 8;
-  if (dk % 8 == 0 && LP <= 64 && (LP & (LP - 1)) == 0 && q_stride % 8 == 0 && al(q) && al(q_norm) && al(k_norm) &&
+  const int LP = dk / 8, n = H * LP + (k ? G * (LP + dv / 8) : 0);  // pieces of a token
+  if (n > kFewPieces && static_cast<long>(rows) * (H + (k ? 2 * G : 0)) > kFewWaves && dk % 8 == 0 && LP <= 64 && (LP & (LP - 1)) == 0 && q_stride % 8 == 0 && al(q) && al(q_norm) && al(k_norm) &&
       nf + nvf <= 4096 &&
       (k == nullptr || (dv % 8 == 0 && k_stride % 8 == 0 && v_stride % 8 == 0 && al(k) && al(v) && al(cache) && koff % 8 == 0 &&
                         voff % 8 == 0 && block_stride % 8 == 0))) {
-    // few tokens: a lane for every piece (64 tokens 3.8 us, 4.6 with 256 lanes); many: smaller workgroups pack better (4,096
-    // tokens 15.4 us, 18.3 with 512)
-    const int threads = std::min(rows <= 1024 ? 512 : 256, (H * LP + (k ? G * (LP + dv / 8) : 0) + 63) / 64 * 64);
-    MIX_DISPATCH(bf, hipLaunchKernelGGL(rope_qkv_cache_wide_kernel<T>, dim3(rows), dim3(threads), (nf + nvf) * sizeof(float2), st,
+    // few tokens: a lane for every piece, over several workgroups where one does not hold them; many: smaller workgroups pack
+    // better (4,096 tokens 15.4 us, 18.3 with 512)
+    const int threads = std::min(rows <= 1024 ? 512 : 256, (n + 63) / 64 * 64);
+    const dim3 grid(rows, rows <= kFewRows ? (n + threads - 1) / threads : 1);
+    MIX_DISPATCH(bf, hipLaunchKernelGGL(rope_qkv_cache_wide_kernel<T>, grid, dim3(threads), (nf + nvf) * sizeof(float2), st,
                                         (T*)q, q_stride, (const T*)k, k_stride, (const T*)v, v_stride, positions, slots,
                                         (T*)cache, block_stride, koff, voff, H, G, dk, dv, bs, freqs, nf, (const T*)q_norm,
                                         (const T*)k_norm, eps, v_freqs, nvf));
@@ -613,8 +620,10 @@ void launch_rope_rows(void* out, long out_stride, const void* x, long x_stride, 
                       int heads, int dim, const float* freqs, int nf, float sign, float scale, bool bf, hipStream_t st) {
   if (rows == 0) return;
   auto al = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  if (dim % 8 == 0 && x_stride % 8 == 0 && out_stride % 8 == 0 && al(x) && al(out) && nf <= 4096) {
-    MIX_DISPATCH(bf, hipLaunchKernelGGL(rope_rows_wide_kernel<T>, dim3(rows), dim3(std::min(256, (heads * dim / 8 + 63) / 64 * 64)), nf * sizeof(float2), st, (T*)out, out_stride,
+  if (static_cast<long>(rows) * heads > kFewWaves && dim % 8 == 0 && x_stride % 8 == 0 && out_stride % 8 == 0 && al(x) && al(out) && nf <= 4096) {
+    const int n = heads * dim / 8, threads = std::min(256, (n + 63) / 64 * 64);
+    const dim3 grid(rows, rows <= kFewRows ? (n + threads - 1) / threads : 1);
+    MIX_DISPATCH(bf, hipLaunchKernelGGL(rope_rows_wide_kernel<T>, grid, dim3(threads), nf * sizeof(float2), st, (T*)out, out_stride,
                                         (const T*)x, x_stride, positions, heads, dim, freqs, nf, sign, scale));
     MXS_CHECK_LAUNCH();
     return;

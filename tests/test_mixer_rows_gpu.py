@@ -70,6 +70,36 @@ def test_rotary_rows(gpu, dt, H, G, dk, dv, nf, nvf, norm):
 
 
 @pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("H,G,dk,dv,nf,nvf", [(6, 3, 16, 24, 8, 12), (32, 8, 64, 64, 32, 0), (5, 5, 64, 40, 9, 20), (128, 8, 128, 128, 64, 0),
+                                              (3, 2, 512, 16, 256, 8), (4, 2, 64, 64, 32, 0), (16, 4, 8, 72, 4, 0)])
+@pytest.mark.parametrize("norm", [False, True])
+def test_rotary_of_many_rows(gpu, dt, H, G, dk, dv, nf, nvf, norm):
+    """Enough tokens and heads for a lane per piece: a token's pieces in one workgroup and over several."""
+    g = torch.Generator().manual_seed(H * dk + nf)
+    bs, koff = 16, 16
+    voff = koff + G * bs * dk
+    for T in (255, 257) if H * dk >= 1024 else (800,):
+        qkv = torch.randn(T, H * dk + G * (dk + dv), generator=g).to(dt)
+        cache = torch.randn(T // bs + 1, voff + G * bs * dv + 8, generator=g).to(dt)
+        pos, slots = torch.arange(T) % 97, torch.randperm(T, generator=g)
+        slots[3] = -1
+        fr, vf = torch.rand(nf, generator=g), torch.rand(nvf, generator=g) if nvf else None
+        qn, kn = ((torch.randn(dk, generator=g)).to(dt) if norm else None for _ in range(2))
+        res = {}
+        for dev in ("cpu", gpu):
+            x, c = qkv.clone().to(dev), cache.clone().to(dev)
+            on = lambda t: None if t is None else t.to(dev)  # noqa: E731
+            q, k, v = x.split([H * dk, G * dk, G * dv], dim=1)
+            seqmix.rope_qkv_cache(q, k, v, on(pos), on(slots), c, koff, voff, H, G, dk, dv, bs, on(fr), on(qn), on(kn), 1e-5, on(vf))
+            y = torch.zeros(T, H * dk + 8, dtype=dt, device=dev)
+            seqmix.rope_rows(q, on(pos), H, dk, on(fr), -1.0, 0.7, y[:, 8:])
+            res[str(dev)] = (x.cpu(), c.cpu(), y.cpu())
+        for a, b in zip(*res.values()):
+            # as above; a rotation of normed entries of up to 5 once more
+            torch.testing.assert_close(a.float(), b.float(), **(dict(rtol=1e-4, atol=4e-4) if dt == torch.float32 else dict(rtol=2.0 ** -6, atol=2.0 ** -5)))
+
+
+@pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("C", [8, 72, 2056])
 @pytest.mark.parametrize("taps", [1, 2, 3, 4, 5])
 @pytest.mark.parametrize("lens", [[1], [8], [9], [1, 1, 1, 1, 1, 1, 1, 1, 1], [3, 4, 1, 2, 17], [7, 1, 8, 16]])
