@@ -28,8 +28,8 @@ void launch_gate_linear(float*, const void*, long, const void*, const void*, int
 void launch_kv_write(void*, long, const void*, long, const void*, long, const int64_t*, int, int, int, int, int, int,
                      int, bool, hipStream_t);
 bool launch_window_attention(void*, const void*, long, const void*, long, const int*, int, const int*, const int*, int,
-                             int, int, int, int, int, int, int, int, float, int, int, int, const float*, int, int, float*,
-                             bool, hipStream_t);
+                             int, int, int, int, int, int, int, int, float, int, int, int, bool, const float*, int, int,
+                             float*, bool, hipStream_t);
 bool launch_matrix_scan(float*, const void*, long, const void*, long, const void*, long, const float*, const float*,
                         float*, long, const int*, long, const int*, const int*, int, int, int, int, int, int, float,
                         float, bool, bool, int, int, float*, float*, long, hipStream_t);
@@ -185,8 +185,11 @@ void window_attention(at::Tensor out, at::Tensor q, at::Tensor cache, at::Tensor
   // a step of few rows, and the long walks of few chunks, split their keys over workgroups
   const int64_t table = block_tables.stride(0) * bs, seen = window > 0 ? window + std::max<int64_t>(keep, 0) : table;
   const int h = static_cast<int>(H), g = static_cast<int>(G);
+  const int64_t span = std::min(max_seq_len > 0 ? std::min(max_seq_len, table) : table, seen);
+  const int max_q = static_cast<int>(std::min<int64_t>(max_query_len, T));
+  const bool by_rows = mxs::row_attention_serves(T, max_q, h, g, span);
   const int nsplit = !bf || dk > 128 || dv > 128 ? 1 :
-      std::min(max_query_len, T) < 16 ? mxs::row_attention_splits(T, h, g, std::min(table, seen)) :
+      by_rows ? mxs::row_attention_splits(T, h, g, std::min(table, seen)) :
       mxs::chunk_attention_splits(T, static_cast<int>(S), h, g, static_cast<int>(dk), static_cast<int>(dv), std::min(max_seq_len, seen));
   at::Tensor part;
   if (nsplit > 1) part = at::empty({T * H * nsplit * (dv + 4)}, out.options().dtype(at::kFloat));
@@ -196,7 +199,7 @@ void window_attention(at::Tensor out, at::Tensor q, at::Tensor cache, at::Tensor
       i32(seq_lens, S, "seq_lens"), static_cast<int>(S), static_cast<int>(T), static_cast<int>(koff),
       static_cast<int>(voff), static_cast<int>(H), static_cast<int>(G), static_cast<int>(dk), static_cast<int>(dv),
       static_cast<int>(bs), static_cast<float>(scale), static_cast<int>(window), static_cast<int>(keep),
-      static_cast<int>(std::min<int64_t>(max_query_len, T)), sinkp, static_cast<int>(v_stride), nsplit,
+      max_q, by_rows, sinkp, static_cast<int>(v_stride), nsplit,
       nsplit > 1 ? part.data_ptr<float>() : nullptr, bf, stream());
   TORCH_CHECK(ok, "window_attention: head sizes beyond what the kernel holds (dv <= 512)");
 }

@@ -43,6 +43,8 @@ bool launch_attention_combine(void* out, const float* part, long rows, int nspli
 // two) tokens a block, value rows vs apart.  nsplit stretches of the keys to a row, fp32 part [rows, H, nsplit, dv + 2] when
 // there are more than one.
 void launch_row_attention(const ChunkArgs& a, int rows, int bs, int vs, int nsplit, float* part, hipStream_t st);
+// whether that form serves a launch whose longest chunk has max_q rows and whose rows see `span` keys at most
+bool row_attention_serves(long rows, int max_q, int H, int G, long span);
 // how many stretches serve rows of at most `span` visible keys
 int row_attention_splits(long rows, int H, int G, long span);
 

@@ -50,8 +50,8 @@ __device__ __forceinline__ float across(float v, bool sum) {  // with the lane 3
 constexpr int kSplitKeys = 768;  // shorter walks are one stretch's alone
 
 // DKP, DVP: head sizes the registers are laid out for (smaller ones ride in zeroed columns); KT: keys of a tile; PAGED:
-// where keys and values are.
-template <int DKP, int DVP, int KT, bool PAGED, bool SPLIT>
+// where keys and values are; WHOLE: a third piece of every weight, all 24 bits.
+template <int DKP, int DVP, int KT, bool PAGED, bool SPLIT, bool WHOLE>
 __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention_kernel(ChunkArgs a) {
   constexpr int KS = DKP / 16, DT = DVP / 32, KU = KT / 32;
   constexpr int KROW = DKP + 8, VROW = DVP + 8;  // padded by 16 bytes: neighbouring rows start in other banks
@@ -256,7 +256,7 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
       const float mneg = m == -INFINITY ? 0.f : -m;  // nothing seen yet: exp2(-inf) stays 0
 #pragma unroll
       for (int n = 0; n < 2 * KU; ++n) {  // 16 keys
-        uint32_t ph[4], pl[4];
+        uint32_t ph[4], pl[4], pr[4];
         float ls = 0.f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -268,6 +268,10 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
           ph[j] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
           const f2_t lo = {p0 - __uint_as_float(u0 & 0xFFFF0000u), p1 - __uint_as_float(u1 & 0xFFFF0000u)};
           pl[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(lo, b2_t));
+          if constexpr (WHOLE) {
+            const f2_t rest = {lo[0] - bf2f_lo(pl[j]), lo[1] - bf2f_hi(pl[j])};
+            pr[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(rest, b2_t));
+          }
         }
         l += ls;
         const b8_t bh = __builtin_bit_cast(b8_t, make_uint4(ph[0], ph[1], ph[2], ph[3]));
@@ -282,6 +286,10 @@ __global__ void __launch_bounds__(256, DKP + DVP <= 128 ? 3 : 2) chunk_attention
           const b8_t vf = __builtin_bit_cast(b8_t, xy);
           o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, bh, o[dt], 0, 0, 0);
           o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, bl, o[dt], 0, 0, 0);
+          if constexpr (WHOLE) {
+            const b8_t br = __builtin_bit_cast(b8_t, make_uint4(pr[0], pr[1], pr[2], pr[3]));
+            o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, br, o[dt], 0, 0, 0);
+          }
         }
       }
     }
@@ -393,14 +401,18 @@ bool launch_chunk_attention(const ChunkArgs& a, int max_q, hipStream_t st) {
   const int n = a.nsplit > 1 ? a.nsplit : 1;
   const dim3 grid(a.G, (static_cast<long>(max_q) * (a.H / a.G) + 127) / 128, a.S * n), block(256);
   if (grid.z > 65535u) return false;
-#define MIX_CHUNK(...)                                                                                                       \
+#define MIX_CHUNK(WHOLE, ...)                                                                                                \
   do {                                                                                                                       \
-    if (n > 1) hipLaunchKernelGGL((chunk_attention_kernel<__VA_ARGS__, true>), grid, block, 0, st, a);                       \
-    else hipLaunchKernelGGL((chunk_attention_kernel<__VA_ARGS__, false>), grid, block, 0, st, a);                            \
+    if (n > 1) hipLaunchKernelGGL((chunk_attention_kernel<__VA_ARGS__, true, WHOLE>), grid, block, 0, st, a);                \
+    else hipLaunchKernelGGL((chunk_attention_kernel<__VA_ARGS__, false, WHOLE>), grid, block, 0, st, a);                     \
   } while (0)
-  if (!paged) MIX_CHUNK(192, 128, 32, false);
-  else if (a.dk <= 64 && a.dv <= 64) MIX_CHUNK(64, 64, 64, true);
-  else MIX_CHUNK(128, 128, 32, true);
+  // chunks of fewer than 16 rows keep all bits of a weight, as the forms for rows do
+  const bool whole = paged && max_q < 16, small = a.dk <= 64 && a.dv <= 64;
+  if (!paged) MIX_CHUNK(false, 192, 128, 32, false);
+  else if (small && whole) MIX_CHUNK(true, 64, 64, 64, true);
+  else if (small) MIX_CHUNK(false, 64, 64, 64, true);
+  else if (whole) MIX_CHUNK(true, 128, 128, 32, true);
+  else MIX_CHUNK(false, 128, 128, 32, true);
 #undef MIX_CHUNK
   MXS_CHECK_LAUNCH();
   return n == 1 || launch_attention_combine(a.out, a.part, static_cast<long>(a.rows) * a.H, n, a.dv, st);

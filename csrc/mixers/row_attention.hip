@@ -250,6 +250,17 @@ int row_attention_splits(long rows, int H, int G, long span) {
   return static_cast<int>(std::max(1L, std::min({static_cast<long>(kMaxSplits), 512 / groups, span / 256})));
 }
 
+// A chunk's rows have workgroups of their own here and read their keys again, in chunk_attention.hip 128 (row, head) pairs share
+// them in one that takes longer to start.  Up to 512 workgroups the rows run side by side; with more, chunks of few rows do too.
+// Rows / chunks, us, 8 kv heads of 64: 4 chunks of 15 7.3 / 8.1, behind 100 keys 8.2 / 9.5, behind 600 15.8 / 20.7; 16 chunks of
+// 5 9.4 / 8.2, 10.3 / 9.6, 23.4 / 20.5, behind 2,000 57 / 29; 64 chunks of 15 53 / 8.5; 64 of 2 behind 600 30.4 / 25.7.  16 rows
+// and more belong to the chunks (behind 2,000 keys 16 rows of 16 heads of 128 take 33 there) but where there is nothing to walk:
+// a chunk of 16 alone 6.4 / 8.1.
+bool row_attention_serves(long rows, int max_q, int H, int G, long span) {
+  const long groups = rows * G * ((H / G + 15) / 16);
+  return max_q <= 1 || (groups < 512 && (max_q < 16 || (max_q < 32 && span <= 64)));
+}
+
 void launch_row_attention(const ChunkArgs& a, int rows, int bs, int vs, int nsplit, float* part, hipStream_t st) {
   int shift = 0;
   while ((1 << shift) < bs) ++shift;

@@ -251,12 +251,12 @@ __global__ void __launch_bounds__(256) window_attention_rows_kernel(
 bool launch_window_attention(void* out, const void* q, long q_stride, const void* cache, long block_stride,
                              const int* block_tables, int bt_stride, const int* qsl, const int* seq_lens, int S,
                              int rows, int koff, int voff, int H, int G, int dk, int dv, int bs, float scale,
-                             int window, int keep, int max_q, const float* sink, int vs, int nsplit, float* part,
+                             int window, int keep, int max_q, bool by_rows, const float* sink, int vs, int nsplit, float* part,
                              bool bf, hipStream_t st) {
   if (rows == 0 || S == 0) return true;
   if (vs <= 0) vs = dv;  // value rows back to back
   // bf16 with heads of whole 16-byte pieces: the matrix-core forms, for prompt chunks (rows of a mixed step's single tokens
-  // ride along as tiles of one row) and for steps of short chunks and single tokens; everything else the forms above
+  // ride along as tiles of one row) and, by_rows, for single tokens and few rows; everything else the forms above
   ChunkArgs a{};
   a.out = (bf16_t*)out;
   a.q = (const bf16_t*)q;
@@ -278,7 +278,7 @@ bool launch_window_attention(void* out, const void* q, long q_stride, const void
   a.nsplit = part ? nsplit : 1;
   a.part = part;
   const bool pieces = bf && dk <= 128 && dv <= 128 && koff % 8 == 0 && voff % 8 == 0 && block_stride % 8 == 0;
-  if (pieces && vs == dv && max_q >= 16 && bs == 16 && dk % 16 == 0 && dv % 16 == 0 && q_stride % 4 == 0 &&
+  if (pieces && !by_rows && vs == dv && bs == 16 && dk % 16 == 0 && dv % 16 == 0 && q_stride % 4 == 0 &&
       reinterpret_cast<uintptr_t>(q) % 8 == 0)
     return launch_chunk_attention(a, max_q, st);
   if (pieces && dk % 8 == 0 && dv % 8 == 0 && vs % 8 == 0 && (bs & (bs - 1)) == 0 && q_stride % 8 == 0 &&

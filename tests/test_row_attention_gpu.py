@@ -76,3 +76,17 @@ def test_blocks_and_value_rows(gpu, bs, vs):
 def test_split_rows(gpu, rows, sink):
     check(gpu, 6, 3, 64, 64, [(37 * i % 900 + (900 if i == 0 else 0), 1) for i in range(rows)], sink=sink, blocks=300)
     check(gpu, 6, 3, 64, 64, [(37 * i % 900, 1) for i in range(rows)], 600, 10, sink=sink, blocks=300)
+
+
+@pytest.mark.parametrize("H,G,dk,dv", [(16, 16, 64, 64), (40, 20, 32, 48), (16, 16, 128, 128), (16, 16, 96, 16)])
+@pytest.mark.parametrize("chunks", [[(0, 5)] * 16, [(20, 2)] * 20, [(0, 15), (33, 1), (100, 2), (62, 3)] * 3, [(2040, 9)] + [(7, 4)] * 10])
+def test_short_chunks_of_many_rows(gpu, H, G, dk, dv, chunks):
+    """More rows and heads than the rows' form takes: chunks of fewer than 16 rows by tiles, weights with all their bits."""
+    check(gpu, H, G, dk, dv, chunks)
+    check(gpu, H, G, dk, dv, chunks, window=9, keep=3, sink=True)
+
+
+@pytest.mark.parametrize("chunks", [[(0, 16)], [(0, 31), (5, 17)], [(33, 31)], [(40, 25)]])
+def test_chunks_with_nothing_to_walk(gpu, chunks):
+    """Chunks of 16 to 31 rows and at most 64 keys, in the rows' form, and just beyond."""
+    check(gpu, 8, 2, 64, 64, chunks, sink=True)
