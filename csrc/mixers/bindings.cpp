@@ -378,7 +378,7 @@ void column_scan(int kind, at::Tensor out, at::Tensor q, at::Tensor k, at::Tenso
   p.unit_eps = static_cast<float>(unit_eps);
   p.piece = 1;
   p.npieces = 1;
-  p.max_q = (max_q == 1 && T == S) ? 1 : 0;  // every sequence brings one row
+  p.max_q = max_q > 1 ? static_cast<int>(std::max<int64_t>(2, std::min(max_q, T))) : max_q == 1 && T == S ? 1 : 0;  // 1: every sequence brings one row
   if (npieces > 1) {  // pieces side by side: scratch [S, npieces, state] twice and the pieces' decays
     TORCH_CHECK(piece >= 16 && sc_local.has_value() && sc_start.has_value() && (delta || sc_decay.has_value()),
                 "a split scan needs its scratch pools");

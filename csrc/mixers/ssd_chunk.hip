@@ -347,11 +347,15 @@ __global__ void __launch_bounds__(256, 2) ssd_chunk_kernel(const ScanArgs p) {
 
 // Whole tiles and 16-byte pieces: state 64 or 128, heads of 32, 64 or 128 that fill a workgroup's 128 columns within a group of
 // B and C.  From 64 rows and 8 rows a sequence on: a chunk of fewer tokens costs what a full one does.  64 heads of 64, state
-// 128, token by token against here: one chunk of 16 tokens 14.6 / 17.6 us, 64 tokens 24.9 / 21.5; 32 chunks of 16 61 / 47;
-// a chunk beside 32 single tokens: of 100 44 / 53, of 200 69 / 64, of 400 122 / 91.
+// 128, token by token against here: one chunk of 64 tokens 22.4 / 17.7 us; 32 chunks of 16 58 / 35; a chunk beside 32 single
+// tokens: of 257 232 / 165, of 400 148 / 111.  Chunks of fewer than 32 tokens only where the heads fill the chip, as token by
+// token they are short walks: 16 chunks of 8, 8 heads 8.8 / 13.8, 32 heads 16.7 / 16.3, 64 heads 27.6 / 21.1; 8 of 24, 8 heads
+// 12.9 / 13.8, 32 heads 17.9 / 14.9; 8 of 32, 8 heads 14.5 / 14.0.
 bool ssd_chunk_fits(const ScanArgs& a, int S) {
   auto al = [](const void* p, long n) { return reinterpret_cast<uintptr_t>(p) % n == 0; };
   const int P = a.dv;
+  const int longest = a.max_q > 1 ? a.max_q : a.n_rows - S + 1;
+  if (longest < 32 && static_cast<long>(a.n_rows) * a.H * P < 1 << 18) return false;
   if (a.n_rows < 64 || a.n_rows < 8L * S || (a.dk != 64 && a.dk != 128) || (P != 32 && P != 64 && P != 128)) return false;
   if ((a.H / a.G) % (128 / P) != 0) return false;
   return a.k_stride % 8 == 0 && a.q_stride % 8 == 0 && a.v_stride % 8 == 0 && al(a.k, 16) && al(a.q, 16) && al(a.v, 16) &&

@@ -58,6 +58,15 @@ def test_chunks(gpu, H, G, N, P, before, new):
     assert torch.equal(pool[:, :4], old[:, :4]) and torch.equal(pool[:, -4:], old[:, -4:])
 
 
+@pytest.mark.parametrize("H,G,N,P", [(64, 1, 128, 64), (64, 8, 64, 64), (32, 1, 64, 128), (2, 1, 128, 64)])
+@pytest.mark.parametrize("before,new", [([0, 9] * 8, [8] * 16), ([3, 0, 1], [31, 30, 31]), ([0, 5] * 4, [9, 12, 1, 31, 8, 20, 2, 17])])
+def test_short_chunks_of_many_heads(gpu, H, G, N, P, before, new):
+    """Chunks of fewer than 32 tokens: in tiles where there are heads enough, token by token for the last line's two."""
+    y, want, st, wst, pool, old, rows = run(gpu, H, G, N, P, before, new, -1.5)
+    torch.testing.assert_close(y, want, rtol=1e-5, atol=1e-4)
+    torch.testing.assert_close(st, wst, rtol=1e-5, atol=1e-4)
+
+
 @pytest.mark.parametrize("a_mean", [-12.0, 3.0, 7.0])
 def test_decays(gpu, a_mean):
     """Half lives of a thousand tokens, and resets within a few or one, where the running sum of exponents is in the thousands."""
