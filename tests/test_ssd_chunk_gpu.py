@@ -58,6 +58,16 @@ def test_chunks(gpu, H, G, N, P, before, new):
     assert torch.equal(pool[:, :4], old[:, :4]) and torch.equal(pool[:, -4:], old[:, -4:])
 
 
+@pytest.mark.parametrize("before,new", [([5] * 9 + [0], [1] * 9 + [512]), ([0, 3, 1, 8], [1, 300, 511, 2]), ([4, 0], [1024, 1])])
+def test_a_spare_piece(gpu, before, new):
+    """Counts of pieces that are multiples of 8: an empty one is put behind them."""
+    piece, n = seqmix._scan_split(len(new), sum(new), max(new), 2 * 128 * 64, 2, 4 * 64, gpu, spare=True)[:2]
+    assert n == -(-max(new) // piece) + 1 and n % 8 == 1
+    y, want, st, wst, *_ = run(gpu, 2, 1, 128, 64, before, new, -1.5)
+    torch.testing.assert_close(y, want, rtol=1e-5, atol=1e-4)
+    torch.testing.assert_close(st, wst, rtol=1e-5, atol=1e-4)
+
+
 @pytest.mark.parametrize("H,G,N,P", [(64, 1, 128, 64), (64, 8, 64, 64), (32, 1, 64, 128), (2, 1, 128, 64)])
 @pytest.mark.parametrize("before,new", [([0, 9] * 8, [8] * 16), ([3, 0, 1], [31, 30, 31]), ([0, 5] * 4, [9, 12, 1, 31, 8, 20, 2, 17])])
 def test_short_chunks_of_many_heads(gpu, H, G, N, P, before, new):
