@@ -486,9 +486,18 @@ def _scan_split(S: int, T: int, max_query_len: int, floats: int, heads: int, dv:
     spare: with several sequences, an empty piece more where the count is a multiple of 8.  Single tokens beside
     a chunk use their first piece only; at strides of 8 states those meet in few channels of the memory (state
     space, 8 heads of 64 x 128, a chunk of 512 beside 64 single tokens: 130 -> 62 us; 500 more tokens: 144 -> 76)."""
+    piece, n = _scan_pieces(S, T, max_query_len, floats, heads, dv, spare)
+    if n == 1:
+        return 1, 1, None, None
+    pool = torch.empty(2, S * n * floats, dtype=torch.float32, device=device)
+    return piece, n, pool[0], pool[1]
+
+
+def _scan_pieces(S: int, T: int, max_query_len: int, floats: int, heads: int, dv: int, spare: bool = False) -> tuple:
+    """(piece, npieces) of _scan_split; npieces 1: not cut."""
     max_query_len = min(max_query_len, T)
     if max_query_len < 128:
-        return 1, 1, None, None
+        return 1, 1
     piece = SCAN_PIECE
     if piece <= 0:
         per_piece = heads * -(-dv // 64) * max(1, T // max_query_len)  # workgroups one piece index adds
@@ -501,10 +510,9 @@ def _scan_split(S: int, T: int, max_query_len: int, floats: int, heads: int, dv:
         if spare and S > 1 and n % 8 == 0 and 2 * S * (n + 1) * floats * 4 <= SCAN_SCRATCH_BYTES:
             n += 1
         if 2 * S * n * floats * 4 <= SCAN_SCRATCH_BYTES:
-            pool = torch.empty(2, S * n * floats, dtype=torch.float32, device=device)
-            return piece, n, pool[0], pool[1]
+            return piece, n
         piece *= 2
-    return 1, 1, None, None
+    return 1, 1
 
 
 def decay_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Tensor, state: torch.Tensor,
@@ -1013,12 +1021,26 @@ def ssd_scan(x: torch.Tensor, B: torch.Tensor, C: torch.Tensor, dt: torch.Tensor
     return out.reshape(T, H * P)
 
 
-# A bf16 step of the delta rule runs in chunks when its longest chunk holds this many tokens, and more for each sequence: token
-# by token a step takes 0.45 us for each token of its longest chunk, in chunks 30 us and 2.7 us a sequence before anything else.
-# 16 heads of 128, token by token / in chunks: one chunk of 64 34 / 42 us, 127 62 / 47, 512 260 / 79, 4,096 1,480 / 437; 32
-# chunks of 16 65 / 97; a chunk beside 32 single tokens: of 200 112 / 115, of 400 203 / 124.
-DELTA_CHUNK_TOKENS, DELTA_CHUNK_TOKENS_PER_SEQ = 64, 6
+# A bf16 step of the delta rule runs in chunks when token by token it would be cut into pieces, and otherwise from
+# DELTA_CHUNK_TOKENS tokens in its longest chunk on, or 32 fewer and so many for each sequence, since a single token costs its
+# heads as much as 32: DELTA_CHUNK_TOKENS_PER_SEQ, or more beside shorter ones where the heads fill the chip (one for each 70,000
+# entries of a sequence's state).  Token by token / in chunks, us, 16 heads of 128: a chunk of 70 39 / 45, 96 49 / 45, 256
+# 177 / 55, 4,096 1,360 / 425; 16 chunks of 100 189 / 172; beside 32 single tokens 128 109 / 129, 257 174 / 142, 400 241 / 149,
+# beside 64 300 242 / 219.  64 heads of 128: beside 32 300 361 / 472, 400 426 / 491, 600 567 / 560.  64 heads of 64: beside 64
+# 300 211 / 239, 512 294 / 276; 16 chunks of 160 294 / 310, as with 16 heads of 128 x 64 148 / 164: such many small heads want
+# some tokens more.
+DELTA_CHUNK_TOKENS, DELTA_CHUNK_TOKENS_PER_SEQ = 96, 5.5
 DELTA_MIN_PIECES = 4  # a split delta-rule scan does three times the work: fewer pieces do not pay
+
+
+def delta_in_chunks(S: int, T: int, max_query_len: int, heads: int, dk: int, dv: int) -> bool:
+    if _scan_pieces(S, T, max_query_len, heads * (dv + dk) * dk, heads, 4 * (dv + dk))[1] >= DELTA_MIN_PIECES:
+        return True
+    each, state = DELTA_CHUNK_TOKENS_PER_SEQ, heads * dk * dv
+    if 2 * T < S * max_query_len:  # mostly shorter ones
+        each = max(each, state / 70000)
+    some = 16 if dk * dv < 128 * 128 <= state / 8 and S > 4 else 0
+    return min(max_query_len, T) >= DELTA_CHUNK_TOKENS + max(0, each * S + some - 32)
 
 
 def delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Tensor, a: torch.Tensor,
@@ -1046,7 +1068,7 @@ def delta_scan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Te
         S = seq_lens.numel()
         args = (out, q, k, v, beta, a, dt_bias, A_log, state, state_rows, int(off), qsl, seq_lens, H, G, dk, dv,
                 float(q_scale), float(unit_eps))
-        if q.dtype == torch.bfloat16 and min(max_query_len, T) >= DELTA_CHUNK_TOKENS + DELTA_CHUNK_TOKENS_PER_SEQ * S:
+        if q.dtype == torch.bfloat16 and delta_in_chunks(S, T, max_query_len, H, dk, dv):
             floats = ext().delta_chunk_floats(dk, dv) * (T // 32 + S) * H
             if 0 < 4 * floats <= SCAN_SCRATCH_BYTES and state.data_ptr() % 16 == 0 and state.stride(0) % 4 == 0 and off % 4 == 0:
                 work = torch.empty(floats, dtype=torch.float32, device=q.device)
