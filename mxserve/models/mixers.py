@@ -87,14 +87,8 @@ class StepContext:
         chunks, nd = getattr(md, "chunks", None), getattr(md, "num_decodes", 0)
         if not chunks or not md.seq_lens.is_cuda or len(chunks) + nd != md.seq_lens.numel():
             return None
-        rows = pairs = 0
-        for past, n in chunks:
-            first = max(past - window + 1, 0) // 16 * 16 if window > 0 else 0
-            rows += past + n - first
-            pairs += n * min(past + (n + 1) // 2, window if window > 0 else 1 << 30)
-        if pairs < EXPAND_MIN_QUERIES * rows or pairs * heads < EXPAND_MIN_PAIRS:
-            return None
-        return seqmix.latent_plan(self.chunk_rows(), md.seq_lens[nd:], window) + (rows,)
+        rows = expanded_rows(chunks, window, heads)
+        return seqmix.latent_plan(self.chunk_rows(), md.seq_lens[nd:], window) + (rows,) if rows else None
 
     def chunk_rows(self) -> torch.Tensor:
         """First rows of the sequences behind the single tokens, counted from the first of them."""
@@ -105,13 +99,34 @@ class StepContext:
 # A latent attention's chunk expands keys and values per head where the gathered rows meet at least this many queries on
 # average.  Per head a key costs 2 * rank * (dim + vdim) operations to expand and every pair of a query and a key
 # 2 * (dim + rot_dim + vdim) instead of the folded form's 2 * (2 rank + rot_dim) (128 + 64, 128, rank 512: 262,144 against
-# 1,536 saved, so from 170 queries on by operations alone); the folded form runs them at a third of the rate as well.  4,096 new
-# tokens, 16 heads of these sizes: 1,142 + 50 us folded (attention, two batched products), 217 + 32 us expanded.
+# 1,536 saved, so from 170 queries on by operations alone); the folded form runs them at a third of the rate as well, and at a
+# tenth for small ranks, so that a rank below the break-even of operations does not make it the better one.  A layer's attention
+# with its projections, folded / expanded, us: 4,096 new tokens, 16 heads, ranks 512 to 64 of 128 + 64, 128 1,243 / 266,
+# 1,665 / 269, 750 / 258, 608 / 257, ranks 64 and 32 of 64 + 32, 64 589 / 236, 516 / 235, 32 heads of 16 + 16, 16, rank 16
+# 783 / 281; 128 behind 2,048, 64 heads of rank 512 203 / 150, 32 heads of rank 64 95 / 67; 64 behind 2,048 133 / 142.
 # It also takes six launches more in a layer (both forms run where single tokens stand beside chunks), which the host pays for
 # in a small step: below this many (query, key, head) triples the folded form's attention is under 70 us (8.5 ps a triple).
+# A walk of few queries and heads leaves the chip idle, and the folded form cuts it finer: beyond EXPAND_SPAN keys the triples grow
+# with them (256 behind 8,192: 4 heads 143 / 155, 8 heads 142 / 141, 16 heads 333 / 210; behind 16,384: 205 / 258, 343 / 290,
+# 606 / 342).
+# Error of the whole layer against 64 bits, folded / expanded, ranks 32 to 512: scores of deviation 1 0.0044 / 0.0038 (512 behind
+# 2,048), 0.0050 / 0.0048 (1,024 tokens); of deviation 4, where single keys decide, 0.0081 / 0.0082 and 0.0089 / 0.0089.
 EXPAND_MIN_QUERIES = 64
 EXPAND_MIN_PAIRS = 8 << 20
+EXPAND_SPAN = 5000
 EXPAND_MAX_BYTES = 1 << 30  # expanded keys and values of a layer; steps with more stay on the folded form
+
+
+def expanded_rows(chunks, window: int, heads: int) -> int:
+    """How many latent rows these (cached, new) chunks gather; 0: the folded form serves them."""
+    rows = pairs = span = 0
+    for past, n in chunks:
+        first = max(past - window + 1, 0) // 16 * 16 if window > 0 else 0
+        rows += past + n - first
+        pairs += n * min(past + (n + 1) // 2, window if window > 0 else 1 << 30)
+        span = max(span, min(past + n, window) if window > 0 else past + n)
+    few = pairs < EXPAND_MIN_QUERIES * rows or pairs * heads < EXPAND_MIN_PAIRS * max(1.0, span / EXPAND_SPAN)
+    return 0 if few else rows
 
 
 class Mixer:
