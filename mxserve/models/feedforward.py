@@ -121,9 +121,12 @@ class RoutedExperts(FeedForward):
     # Sorted rows: an expert's own two products take no less than about 40 us, however few its rows (and half as long again as
     # its share of a batched product when it has a thousand: they fill a third of the chip).  8 experts of 2,048 x 2,560,
     # even choices, products alone: 64 tokens 333 us one by one, 49 us in slabs; 512 tokens 332 / 80; 2,048: 353 / 141;
-    # 4,096: 435 / 273.  So slabs, until their empty rows (at a large product's rate) and the weights of experts without rows
-    # (at the memory's) cost more than 30 us for each expert that has some.
+    # 4,096: 435 / 273.  So slabs, until their empty rows (at a large product's rate, and read and written by two products and the
+    # activation at the memory's) and the weights of experts without rows cost more than 30 us for each expert that has some: 128
+    # experts of 128 x 64, 4,096 tokens with one of them 102 us one by one, 240 in slabs; 8 of 256 x 512, 8,192 tokens with two
+    # of them 155 / 193.  And never more than SLAB_MAX_BYTES of slabs, however the rows fall.
     SLAB_GAIN_S, SLAB_FLOPS, SLAB_BYTES = 30e-6, 1e15, 5e12
+    SLAB_MAX_BYTES = 2 << 30
 
     def __init__(self, prefix: str, width: int, experts: int, top: int, ff: int, limit: Optional[float],
                  shared: Optional[FeedForward] = None, alpha: float = 1.702, renorm: bool = False,
@@ -207,6 +210,18 @@ class RoutedExperts(FeedForward):
                                  correction=w[p + "correction"] if self.correction else None, groups=self.groups,
                                  keep=self.keep, scale=self.scale) + (None,)
 
+    def slab_rows(self, offs: list, size: int) -> int:
+        """Rows of an expert's slab for these offsets of sorted rows; 0: one product pair per expert."""
+        counts = [b - a for a, b in zip(offs, offs[1:])]
+        cap, used = max(counts), self.E - counts.count(0)
+        up = 2 * self.ff if self.gated else self.ff
+        per_row = self.width * (up + self.ff)  # multiply-adds of a row, weights of an expert
+        row = 2 * self.width + up + self.ff  # what a row takes in memory; the up product's output is read once more, as is the rest
+        empty = self.E * cap - offs[-1]
+        cost = (2.0 * per_row * empty / self.SLAB_FLOPS
+                + size * (2.0 * (row - self.width) * empty + per_row * (self.E - used)) / self.SLAB_BYTES)
+        return cap if cost <= self.SLAB_GAIN_S * used and self.E * cap * row * size <= self.SLAB_MAX_BYTES else 0
+
     def rows(self, h: torch.Tensor, w: dict) -> seqmix.ExpertRows:
         """The experts' outputs and what sums them: for a layer whose stream update takes the sum itself."""
         p, T = self.p, h.shape[0]
@@ -226,11 +241,8 @@ class RoutedExperts(FeedForward):
                                      gate=gate)
         offs, inv = seqmix.expert_align(ids, self.E)
         o = offs.tolist()  # the one host read of this path
-        counts = [b - a for a, b in zip(o, o[1:])]
-        cap, used = max(counts), sum(n > 0 for n in counts)
-        per_row = up[0].numel() + down[0].numel()  # multiply-adds of a row, weights of an expert
-        if (2.0 * per_row * (self.E * cap - o[-1]) / self.SLAB_FLOPS
-                + per_row * up.element_size() * (self.E - used) / self.SLAB_BYTES) <= self.SLAB_GAIN_S * used:
+        cap = self.slab_rows(o, up.element_size())
+        if cap:
             xs, index = seqmix.gather_slabs(h, w_in, ids, offs, inv, cap)
             a = self.act(torch.bmm(xs, up).view(self.E * cap, -1))
             ys = torch.bmm(a.view(self.E, cap, -1), down)

@@ -77,3 +77,17 @@ def test_capped(gpu, dt, F, pad):
     gu[0, 0], gu[1, F] = float("inf"), float("-inf")
     got, want = seqmix.capped_glu(gu.to(gpu), 7.0), seqmix.capped_glu(gu, 7.0)
     torch.testing.assert_close(got.cpu().float(), want.float(), **(dict(rtol=1e-5, atol=1e-5) if dt == torch.float32 else dict(rtol=2.0 ** -7, atol=1e-5)))
+
+
+@pytest.mark.parametrize("E,top,W,ff,counts,slabs", [
+    (8, 2, 2048, 2560, [16] * 8, True), (8, 2, 2048, 2560, [1024] * 8, True), (8, 2, 2048, 2560, [4096, 4096] + [0] * 6, False),
+    (128, 1, 128, 64, [4096] + [0] * 127, False), (128, 1, 128, 64, [32] * 128, True), (8, 2, 256, 512, [8192, 8192] + [0] * 6, False),
+    (8, 2, 256, 512, [300, 212] + [0] * 6, True), (64, 6, 2048, 1408, [96] * 64, True), (8, 2, 4096, 7168, [8192] * 8, False)])
+def test_when_slabs_pay(E, top, W, ff, counts, slabs):
+    """Neither many empty rows, however few their operations, nor more memory than SLAB_MAX_BYTES."""
+    offs = [0]
+    for n in counts:
+        offs.append(offs[-1] + n)
+    cap = RoutedExperts("", W, E, top, ff, 7.0).slab_rows(offs, 2)
+    assert cap == (max(counts) if slabs else 0)
+    assert E * cap * (2 * W + 3 * ff) * 2 <= RoutedExperts.SLAB_MAX_BYTES
