@@ -177,7 +177,7 @@ struct MemRow {
 // 128k row) are collected and ranked against each other; a fuller bin is cut again.  Two passes over the row where a
 // bisection over value took 32, each with an exponential per logit: that was what a row's time went into, and a row is
 // one workgroup, so a step with few sampled rows waits for it (MI355X, 128,256 bf16 logits, 13 rows: 275 us; 32,000
-// fp32 logits, 64 rows: 177 us.  Now 82 us and 27 us).  Shares (at most 1) are 2^-46 fixed point, what 64-bit sums of
+// fp32 logits, 64 rows: 177 us.  Now 61 us and 23 us).  Shares (at most 1) are 2^-46 fixed point, what 64-bit sums of
 // 2^17 of them hold, with a bit less for each doubling of the row beyond: the sums do not depend on the order of the LDS
 // atomics, so a request's tokens stay reproducible.  A share loses less than a step, a row 2^-29 of its sum, where an fp32
 // sum rounds at 2^-24 (one word of 32 bits a share, 2^-15 of a row: 2 us less of 60).

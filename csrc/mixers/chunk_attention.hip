@@ -14,8 +14,9 @@
 // exponentials, and 24 matrix instructions, and the two kinds hardly overlap (interleaving them by hand, four waves a SIMD,
 // walks paired long with short, and walks that begin at different keys all measured the same or slower).
 // 4,096 rows, 32 heads of 64 over 8 kv heads: 1,127 us with one wave per 16 rows of a head on the 16-wide instructions and
-// 2-byte reads of V (the form that this one replaced), 139 us; window 1,024: 75 us; 16 heads of 128: 192 us.  Keys of 128 + 64 and values of 128 expanded from latent rows of 576, 16 heads,
-// 4,096 rows: 217 us and 50 us for gathering and expanding, against 1,142 us over the rows themselves with folded queries.
+// 2-byte reads of V (the form that this one replaced), 125 us; window 1,024: 72 us; 16 heads of 128: 192 us.  Keys of 128 + 64
+// and values of 128 expanded from latent rows of 576, 16 heads, 4,096 rows: 189 us and 50 us for gathering and expanding, against
+// 1,142 us over the rows themselves with folded queries.
 #include "chunk_attention.h"
 #include "chunk_walk.h"
 #include "mix_common.h"

@@ -17,8 +17,10 @@
 // exponents; gated linear attention: the summed logarithms per key channel; delta rule: the piece's dk x dk transition matrix, from dk more columns started as the
 // identity); the states at the pieces' starts are chained from those; pass 2 runs every piece again
 // from its true start and writes the outputs.
-// A token's sums run in an order fixed by the sizes alone, so cutting a prompt differently gives the
-// same bits.  State, decays, gates and every product are fp32; the operands come as bf16 or fp32.
+// A token's sums run in an order fixed by the sizes alone: uncut walks of one prompt in other parts give the same bits.  Long
+// bf16 chunks of the state space and the delta rule go by tiles counted from a part's first token (ssd_chunk.hip,
+// delta_chunk.hip), so there, as with pieces, the cut changes the order of fp32 sums.  State, decays, gates and every product
+// are fp32; the operands come as bf16 or fp32.
 #include <algorithm>
 #include <type_traits>
 
