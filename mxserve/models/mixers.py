@@ -642,7 +642,8 @@ class LatentAttention(Mixer):
         dq, nd = self.dn + self.dr, getattr(md, "num_decodes", 0)
         plan = None
         if dq <= 192 and dq % 16 == 0 and self.vd <= 128 and self.vd % 16 == 0 and self.dn % 8 == 0 and self.dr % 8 == 0 and \
-                self.rank % 8 == 0 and koff % 8 == 0 and ctx.cache.shape[1] % 8 == 0 and ctx.block_size == 16:
+                self.rank % 8 == 0 and koff % 8 == 0 and ctx.cache.stride(0) % 8 == 0 and ctx.cache.data_ptr() % 16 == 0 and \
+                ctx.block_size == 16:
             plan = ctx.expansion(self.window, H)
         if plan is None or 2 * plan[2] * H * (self.dn + self.vd) > EXPAND_MAX_BYTES:
             return False

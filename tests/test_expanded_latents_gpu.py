@@ -185,3 +185,29 @@ def test_a_value_reaches_only_queries_that_see_it(gpu, past, new, window):
         assert not torch.isfinite(y[seen, 1, 5]).any()
         y[seen, 1, 5] = clean.view(new, H, dv)[seen, 1, 5]
         torch.testing.assert_close(y.view(new, -1), clean, rtol=2.0 ** -7, atol=2.0 ** -12)
+
+
+def test_pages_off_the_16_byte_grid_fold(gpu, monkeypatch):
+    """Pages that the gathering kernel does not take are served by the folded form, as before there was another."""
+    monkeypatch.setattr(mixers, "EXPAND_MIN_QUERIES", 0)
+    monkeypatch.setattr(mixers, "EXPAND_MIN_PAIRS", 0)
+    W, H, T, rot = 128, 2, 80, {"dims": 32, "base": 10000.0}
+    m = LatentAttention("", W, H, 64, 32, 64, 64, 64, 96 ** -0.5, rot)
+    g = torch.Generator().manual_seed(3)
+    names = m.proj_rows()
+    w = {k: (torch.randn(s, generator=g) * s[-1] ** -0.5).bfloat16().to(gpu) for k, s in
+         {**{k: (r, W) for k, r in names}, **m.extra_shapes()}.items()}
+    h = torch.randn(T, W, generator=g).bfloat16().to(gpu)
+    y = h @ torch.cat([w.pop(k) for k, _ in names]).T
+    m.finish_weights(w)
+    pos = torch.arange(T, device=gpu)
+    ints = [torch.tensor(x, dtype=torch.int32, device=gpu) for x in ([[0, 1, 2, 3, 4]], [0, T], [T])]
+    md = types.SimpleNamespace(positions=pos, slot_mapping=pos, block_tables=ints[0], query_start_loc=ints[1],
+                               prefill_query_start_loc=ints[1], seq_lens=ints[2], max_query_len=T, max_seq_len=T, num_decodes=0,
+                               chunks=((0, T),))
+    outs = []
+    for shift in (0, 4):
+        cache = torch.zeros(5 * 16 * m.dk + 8, dtype=torch.bfloat16, device=gpu)[shift:shift + 5 * 16 * m.dk].view(5, -1)
+        outs.append(m.forward([y[:, :64], y[:, 64:]], h, w, StepContext(md=md, cache=cache, state=None, block_size=16, eps=1e-5), 0, 0, 0))
+    # both forms round queries or keys, values and outputs to bf16: some 2^-8 of the layer's scale
+    assert float((outs[0] - outs[1]).float().norm() / outs[0].float().norm()) < 0.012
