@@ -163,7 +163,7 @@ def test_mixer_expands_and_folds(gpu, monkeypatch, window, singles):
     want = torch.cat(want) @ d["o"].T
     err = {k: float((o - want).norm() / want.norm()) for k, o in outs.items()}
     # the chain of bf16 roundings (projections, rows, keys, values, outputs): about six of 2^-9 each
-    assert err["folded"] < 0.012 and err["expanded"] < 0.012 and err["expanded"] < 1.2 * err["folded"], err
+    assert err["folded"] < 0.012 and err["expanded"] < 0.012 and err["expanded"] <= err["folded"], err
 
 
 @pytest.mark.parametrize("past,new,window", [(0, 140, 0), (75, 130, 50)])
